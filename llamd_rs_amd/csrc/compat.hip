@@ -282,26 +282,109 @@ __global__ __launch_bounds__(64) void softmax_rows(const float *x, float *o, int
 }
 
 // CpuBackend::matmul (lib.rs:126-149): out[j * m + i] = sum over t in order
-// of w[i][t] * x[j][t], from 0.0, unfused. One thread per output element;
-// the 64 rows of a wave read their w rows through LDS in 64-wide k strips.
-__global__ __launch_bounds__(64) void matmul_f32_seq(const float *w, const float *x, float *out,
-                                                     int m, int n, int k) {
-    __shared__ float ws[64][65];
-    const int lane = threadIdx.x;
-    const int i0 = blockIdx.x * 64, j = blockIdx.y;
-    const float *xr = x + (size_t)j * k;
-    float acc = 0.0f;
-    for (int t0 = 0; t0 < k; t0 += 64) {
-        const int kt = min(64, k - t0);
-        for (int r = 0; r < 64; ++r) {
-            const int i = i0 + r;
-            ws[r][lane] = (i < m && lane < kt) ? w[(size_t)i * k + t0 + lane] : 0.0f;
+// of w[i][t] * x[j][t], from 0.0, unfused. A wave forms 64 rows x RN columns,
+// one row per lane and RN running sums in registers; the workgroup's four
+// waves take four column groups of the same 64 rows. The rows reach LDS 32
+// values of k at a time (the next strip's loads in flight under the sums) and
+// each lane reads its own row, four values per read; a column's values are
+// the same for the whole wave, so they come through the scalar cache into
+// SGPRs, G of them a group ahead of their use.
+// Bound: the multiply and the add of every term, which the reference rounds
+// apart: 43 us of vector issue at 2048 x 200 x 2048 (m, n, k), which takes 64-72
+// us; one output per thread and a serial staging loop took 750-1030. Where the
+// waves do not fill the SIMDs (n = 1: 30 us, 248 before) the chain of k
+// dependent adds and the strip's round trip through LDS are what is left.
+// Columns' values by DPP (row_newbcast) from vector registers instead of
+// SGPRs: 73-78 us at that size (the DPP multiply issues at a lower rate);
+// 4..7 columns per wave spill SGPRs: 71-204 us.
+constexpr int MM_KT = 32;            // k per LDS strip
+constexpr int MM_LD = MM_KT + 4;     // padded row (conflict-free 16-byte reads)
+// 16 bytes of a row whose length need not be a multiple of 4
+typedef float mm_f4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef const __attribute__((address_space(4))) float *mm_cptr;
+
+template <int RN>
+__global__ __launch_bounds__(256) void matmul_f32_seq(const float *w, const float *x, float *out,
+                                                      int m, int n, int k) {
+    __shared__ __align__(16) float ws[2][64 * MM_LD];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i0 = blockIdx.x * 64, j0 = (blockIdx.y * 4 + wave) * RN;
+    mm_cptr xr[RN];
+#pragma unroll
+    for (int r = 0; r < RN; ++r) xr[r] = (mm_cptr)(x + (size_t)min(j0 + r, n - 1) * k);
+    float acc[RN];
+#pragma unroll
+    for (int r = 0; r < RN; ++r) acc[r] = 0.0f;
+    // this thread's share of a strip: 8 values of row i0 + tid / 4
+    const int srow = tid >> 2, sk = (tid & 3) * 8;
+    const float *wr = w + (size_t)min(i0 + srow, m - 1) * k;
+    mm_f4 s0, s1;
+    const auto load = [&](int t0) {
+        if (t0 + MM_KT <= k) {
+            s0 = *(const mm_f4 *)(wr + t0 + sk);
+            s1 = *(const mm_f4 *)(wr + t0 + sk + 4);
+        } else {  // the last, partial strip: values past k are not used
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s0[e] = wr[min(t0 + sk + e, k - 1)];
+                s1[e] = wr[min(t0 + sk + 4 + e, k - 1)];
+            }
         }
+    };
+    load(0);
+    // the columns' values of G positions of k, a group ahead of their use
+    constexpr int G = RN == 1 ? 16 : RN == 2 ? 8 : 4;
+    float xa[RN][G], xb[RN][G];
+    const auto xload = [&](float (&xs)[RN][G], int t) {
+#pragma unroll
+        for (int r = 0; r < RN; ++r)
+#pragma unroll
+            for (int e = 0; e < G; ++e) xs[r][e] = xr[r][t + e];
+    };
+    const auto sums = [&](const float (&xs)[RN][G], const float *wv) {
+#pragma unroll
+        for (int e = 0; e < G; ++e)
+#pragma unroll
+            for (int r = 0; r < RN; ++r) acc[r] = acc[r] + wv[e] * xs[r][e];
+    };
+    if (k >= MM_KT) xload(xa, 0);
+    for (int t0 = 0, buf = 0; t0 < k; t0 += MM_KT, buf ^= 1) {
+        float *dst = ws[buf] + srow * MM_LD + sk;
+        *(float4 *)dst = make_float4(s0[0], s0[1], s0[2], s0[3]);
+        *(float4 *)(dst + 4) = make_float4(s1[0], s1[1], s1[2], s1[3]);
+        // one barrier per strip: the buffer written next was last read before
+        // the barrier of the strip between
         __syncthreads();
-        for (int t = 0; t < kt; ++t) acc = acc + ws[lane][t] * xr[t0 + t];
-        __syncthreads();
+        if (t0 + MM_KT < k) load(t0 + MM_KT);
+        const float *row = ws[buf] + lane * MM_LD;
+        if (t0 + MM_KT <= k) {
+            float wv[MM_KT];
+#pragma unroll
+            for (int t = 0; t < MM_KT; t += 4) *(float4 *)(wv + t) = *(const float4 *)(row + t);
+            // past the last full strip the loads re-read it, unused
+            const int next = t0 + 2 * MM_KT <= k ? t0 + MM_KT : t0;
+#pragma unroll
+            for (int t = 0; t < MM_KT; t += 2 * G) {
+                xload(xb, t0 + t + G);
+                __builtin_amdgcn_sched_barrier(0);
+                sums(xa, wv + t);
+                xload(xa, t + 2 * G < MM_KT ? t0 + t + 2 * G : next);
+                __builtin_amdgcn_sched_barrier(0);
+                sums(xb, wv + t + G);
+            }
+        } else {
+            for (int t = 0; t < k - t0; ++t) {
+                const float wv = row[t];
+#pragma unroll
+                for (int r = 0; r < RN; ++r) acc[r] = acc[r] + wv * xr[r][t0 + t];
+            }
+        }
     }
-    if (i0 + lane < m) out[(size_t)j * m + i0 + lane] = acc;
+    if (i0 + lane < m)
+#pragma unroll
+        for (int r = 0; r < RN; ++r)
+            if (j0 + r < n) out[(size_t)(j0 + r) * m + i0 + lane] = acc[r];
 }
 
 }  // namespace
@@ -394,10 +477,39 @@ int launch_softmax_rows(const float *x, float *o, int rows, int n, hipStream_t s
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+// Columns per wave. Measured at k = 2048 (us): a wave alone on its SIMD takes
+// 30 / 44 / 47 with 1 / 2 / 3 columns; SIMDs with w waves each take 10.3 w /
+// 16 w / 21.3 w. The smallest of the three for the waves the shape makes.
+static int matmul_cols(int m, int n) {
+    const double alone[3] = {30, 44, 47}, shared[3] = {10.3, 16, 21.3};
+    int best = 1;
+    double cost = 1e30;
+    for (int rn = 1; rn <= 3; ++rn) {
+        const long waves = (long)((m + 63) / 64) * ((n + rn - 1) / rn);
+        const double c = std::max(alone[rn - 1], shared[rn - 1] * (double)((waves + 1023) / 1024));
+        if (c < cost) {
+            cost = c;
+            best = rn;
+        }
+    }
+    return best;
+}
+
+template <int RN>
+static void matmul_go(const float *w, const float *x, float *out, int m, int n, int k,
+                      hipStream_t st) {
+    hipLaunchKernelGGL(matmul_f32_seq<RN>, dim3((m + 63) / 64, (n + 4 * RN - 1) / (4 * RN)),
+                       dim3(256), 0, st, w, x, out, m, n, k);
+}
+
 int launch_matmul_f32_seq(const float *w, const float *x, float *out, int m, int n, int k,
                           hipStream_t st) {
     if (m <= 0 || n <= 0 || k <= 0 || n > 65535) return -1;
-    hipLaunchKernelGGL(matmul_f32_seq, dim3((m + 63) / 64, n), dim3(64), 0, st, w, x, out, m, n, k);
+    switch (matmul_cols(m, n)) {
+        case 1: matmul_go<1>(w, x, out, m, n, k, st); break;
+        case 2: matmul_go<2>(w, x, out, m, n, k, st); break;
+        default: matmul_go<3>(w, x, out, m, n, k, st); break;
+    }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
