@@ -440,6 +440,18 @@ void attend(const float *q, const float *kc, const float *vc, float *out, int n_
     REFUSE_IF(max_kv > attend_max_kv() || n_kv > attend_max_kv(),
               "attention: at most %d positions (asked %d)", attend_max_kv(), std::max(max_kv, n_kv));
     const float scale = 1.0f / sqrtf((float)hd);  // attention.rs:87
+    // what one sequence can hold: all of the kernels' range when the position
+    // is on the device and only this cache is read, else its slice
+    const int cap = !pos ? n_kv : nseq == 1 ? attend_max_kv() : max_kv;
+    if (attend_split_fits(n_head, n_head_kv, hd, cap)) {
+        std::lock_guard<std::mutex> lk(g_smu);
+        float *scores = (float *)scratch(attend_split_scores(n_head, cap, nseq) * 4);
+        if (!scores) return fwd_refused();
+        if (launch_attend_split(q, kc, vc, pos, n_head, n_head_kv, hd, scale, cap, scores, out, S(), nseq,
+                                n_kv, pos_stride, (size_t)max_kv * n_head_kv * hd, pos ? max_kv : n_kv))
+            REFUSE("attention: launch");
+        return;
+    }
     if (launch_attend_decode(q, kc, vc, pos, n_head, n_head_kv, hd, scale, out, S(), nseq, n_kv,
                              pos_stride, (size_t)max_kv * n_head_kv * hd))
         REFUSE("attention: launch");

@@ -6,6 +6,8 @@
 //
 // The token and position are read from device memory (not kernel
 // arguments), so a step's launches do not change from token to token.
+#include <algorithm>
+
 #include "common.hpp"
 #include "exact_sum.hpp"
 #include "expf_ref.h"
@@ -442,190 +444,430 @@ __global__ __launch_bounds__(512) void attend_fused(
     }
 }
 
-// ---- attention over long contexts: logits spread over the GPU -------------
-// attend_fused runs n_head / 2 workgroups and walks the positions 64 at a
-// time, so its cost grows by ~50 ns per position and layer. Past a few
-// hundred positions the same arithmetic runs in two launches instead (after
-// qk_norm_rope_store has put the normed, rotated Q in place and K, V in the
-// cache, and before the Q8_K of the output: q8k_quantize, or inside the O
-// projection, q6k_mv_f32x):
-//  - attend_logits: workgroup w keeps kv head w % n_head_kv and takes its
-//    position blocks w / n_head_kv, + gridDim.x / n_head_kv, ...; the block's
-//    K rows are staged in LDS (rows padded to 132 floats) and thread
-//    (query head j of the group, position t) forms logit_t = (q . k_t, the
-//    128 products added in order from 0) * scale into scores.
-//  - attend_finish: AF_SL 1024-thread workgroups per head, each on
-//    128 / AF_SL dimensions: max (order free), e_t = expf(logit_t - max),
-//    their in-order sum by exact_sum_nonneg (the reference's bits from a
-//    workgroup-wide certificate), inv = 1 / sum (every workgroup of the head
-//    the same), then one thread per dimension adds (e_t * inv) * v_t[d] in
-//    position order from V rows staged in LDS (half a row per position)
-//    into the f32 output.
-// The same operations in the same order as attend_fused (and the reference,
+// ---- attention split over the GPU -------------------------------------------
+// attend_fused and attend_decode give a head one workgroup that walks its
+// positions, so their cost grows by 50-70 ns per position. Here the same
+// arithmetic runs in one or two launches, for any number of sequences (Q
+// normed and rotated and K, V already in the cache):
+//  - attend_scores (past a.fuse positions): a workgroup takes 64 positions of
+//    one kv head, one wave per query head of its group, one lane per position.
+//    The K rows are staged in LDS once for the group; the wave's q comes
+//    through the scalar cache into SGPRs, so the in-order 128-term dot reads
+//    LDS once per four terms.
+//  - attend_mix: a workgroup per head and slice of DS dimensions: the logits
+//    (read, or formed from K rows staged in LDS), their max (order free), e_t =
+//    expf(logit_t - max), the in-order sum of e_t (one lane, or past
+//    ATT_SERIAL terms exact_sum_nonneg: the reference's bits from a
+//    workgroup-wide certificate), w_t = e_t * (1 / sum), then out[d] =
+//    sum_t w_t * v_t[d] in position order.
+// The last sum is one dependent chain of n_kv adds per output and bounds the
+// kernel. So the folding waves (one lane per dimension) do nothing but read
+// four products and add them: other waves load V a few chunks ahead, multiply
+// by the weights and hand chunks of products over in LDS, transposed so that a
+// lane's four next products are one read. What is left is the chain itself, 3.6
+// ns per position, and about 1.2 ns of waiting for the products; a barrier per
+// 32 positions instead of 128 (64 where CUs are shared) costs another 2-4 ns.
+// The same operations in the same order as attend_decode (and the reference,
 // attention.rs:73-125): the same bits.
-constexpr int AL_KS = ATT_HD + 4;   // padded K row in LDS
-constexpr int AL_MAX_GROUP = 16;    // query heads per kv head
+constexpr int AS_POS = 64;          // positions per block of attend_scores
+constexpr int AS_MAX_GROUP = 16;    // query heads per kv head
+constexpr int ATT_SERIAL = 320;     // e_t that one lane adds
 
-__global__ __launch_bounds__(256) void attend_logits(const float *q, const float *kc,
-                                                     const int32_t *pos_p, int n_head,
-                                                     int n_head_kv, float scale, float *scores,
-                                                     int max_kv) {
-    constexpr int HD = ATT_HD;
-    __shared__ __align__(16) float ks[64 * AL_KS];
-    __shared__ __align__(16) float qs[AL_MAX_GROUP * HD];
-    const int group = n_head / n_head_kv;
-    const int ppi = min(64, 256 / group);  // positions per block
-    const int g = blockIdx.x % n_head_kv;
-    const int stride = gridDim.x / n_head_kv;
-    const int kv_dim = n_head_kv * HD;
-    const int n_kv = pos_p[0] + 1;
-    const int nb = (n_kv + ppi - 1) / ppi;
-    const int tid = threadIdx.x;
-    if ((int)blockIdx.x / n_head_kv >= nb) return;
-    for (int i = tid; i < group * HD / 4; i += 256)
-        *(float4 *)(qs + 4 * i) = *(const float4 *)(q + (size_t)g * group * HD + 4 * i);
-    const int hl = tid / ppi, tl = tid - hl * ppi;
-    for (int pb = blockIdx.x / n_head_kv; pb < nb; pb += stride) {
-        const int t0 = pb * ppi, np = min(ppi, n_kv - t0);
+typedef const __attribute__((address_space(4))) float *att_cptr;
+
+struct AttArgs {
+    const float *q, *kc, *vc;
+    const int32_t *pos_p;     // n_kv = pos_p[s * pos_stride] + 1 (null: n_kv_fixed)
+    float *scores;            // [nseq][n_head][cap]
+    float *out;               // [nseq][n_head * HD]
+    size_t seq_stride;        // floats between two sequences' caches
+    int pos_stride, n_kv_fixed, n_head, n_head_kv, cap, fuse, grid_x;
+    float scale;
+};
+
+__device__ __forceinline__ int att_n_kv(const AttArgs &a, int s) {
+    return a.pos_p ? a.pos_p[(size_t)s * a.pos_stride] + 1 : a.n_kv_fixed;
+}
+
+// One word of each of q's 64-byte lines, so that the scalar cache holds them
+// when the dot products read the rest.
+template <int HD>
+__device__ __forceinline__ void att_touch(att_cptr q) {
+#pragma unroll
+    for (int d = 0; d < HD; d += 16) asm volatile("" ::"s"(q[d]));
+}
+
+template <int HD>
+__global__ __launch_bounds__(64 * AS_MAX_GROUP) void attend_scores(AttArgs a) {
+    constexpr int KS = HD + 4;  // padded row: conflict-free 16-byte reads
+    __shared__ __align__(16) float ks[AS_POS * KS];
+    const int group = a.n_head / a.n_head_kv, nt = 64 * group;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = blockIdx.y, s = blockIdx.z;
+    const int n_kv = att_n_kv(a, s), kv_dim = a.n_head_kv * HD;
+    if (n_kv <= a.fuse || n_kv > a.cap) return;
+    const int head = s * a.n_head + g * group + wave;
+    const att_cptr q = (att_cptr)(a.q + (size_t)head * HD);
+    const float *kc = a.kc + (size_t)s * a.seq_stride + (size_t)g * HD;
+    for (int t0 = blockIdx.x * AS_POS; t0 < n_kv; t0 += a.grid_x * AS_POS) {
+        const int np = min(AS_POS, n_kv - t0);
         __syncthreads();  // the previous block's rows are read
-        for (int i = tid; i < np * (HD / 4); i += 256) {
-            const int t = i / (HD / 4), d4 = i - t * (HD / 4);
-            *(float4 *)(ks + t * AL_KS + 4 * d4) =
-                *(const float4 *)(kc + (size_t)(t0 + t) * kv_dim + (size_t)g * HD + 4 * d4);
+        for (int i0 = tid; i0 < np * (HD / 4); i0 += 4 * nt) {
+            att_f4 r[4];  // four loads in flight; those past the block re-read its last row
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int i = i0 + k * nt, t = min(i / (HD / 4), np - 1);
+                r[k] = *(const att_f4 *)(kc + (size_t)(t0 + t) * kv_dim + 4 * (i % (HD / 4)));
+            }
+            if (t0 == (int)blockIdx.x * AS_POS && i0 == tid) att_touch<HD>(q);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int i = i0 + k * nt, t = i / (HD / 4);
+                if (t < np) *(att_f4 *)(ks + t * KS + 4 * (i % (HD / 4))) = r[k];
+            }
         }
         __syncthreads();
-        if (hl < group && tl < np) {
-            const float *kr = ks + tl * AL_KS, *qr = qs + hl * HD;
-            float dot = 0.0f;
+        const float *kr = ks + lane * KS;
+        float dot = 0.0f;
 #pragma unroll
-            for (int d0 = 0; d0 < HD; d0 += 32) {
-                float4 k4[8], q4[8];
+        for (int d0 = 0; d0 < HD; d0 += 16) {
+            att_f4 k4[4];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    k4[j] = *(const float4 *)(kr + d0 + 4 * j);
-                    q4[j] = *(const float4 *)(qr + d0 + 4 * j);
-                }
+            for (int j = 0; j < 4; ++j) k4[j] = *(const att_f4 *)(kr + d0 + 4 * j);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    dot = dot + q4[j].x * k4[j].x;
-                    dot = dot + q4[j].y * k4[j].y;
-                    dot = dot + q4[j].z * k4[j].z;
-                    dot = dot + q4[j].w * k4[j].w;
-                }
-            }
-            scores[(size_t)(g * group + hl) * max_kv + t0 + tl] = dot * scale;
+            for (int j = 0; j < 16; ++j) dot = dot + q[d0 + j] * k4[j / 4][j % 4];
         }
+        if (lane < np) a.scores[(size_t)head * a.cap + t0 + lane] = dot * a.scale;
     }
 }
 
-constexpr int AF_PER = 8;  // float4s of one V chunk per thread
-constexpr int AF_SL = 2;   // workgroups per head (dimension slices)
-constexpr int AF_DS = ATT_HD / AF_SL;
+// The logit of one position for one head, q through the scalar cache.
+template <int HD>
+__device__ __forceinline__ float att_logit(const float *qp, const float *kr, float scale) {
+    att_cptr q = (att_cptr)qp;
+    asm volatile("" : "+s"(q));  // read again for each position: 128 registers otherwise
+    float dot = 0.0f;
+#pragma unroll
+    for (int d0 = 0; d0 < HD; d0 += 32) {
+        att_f4 k4[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) k4[j] = *(const att_f4 *)(kr + d0 + 4 * j);
+#pragma unroll
+        for (int j = 0; j < 32; ++j) dot = dot + q[d0 + j] * k4[j / 4][j % 4];
+    }
+    return dot * scale;
+}
 
-__global__ __launch_bounds__(1024) void attend_finish(const float *scores, const float *vc,
-                                                      const int32_t *pos_p, int n_head,
-                                                      int n_head_kv, int max_kv, int chunk,
-                                                      float *out) {
-    constexpr int HD = ATT_HD, DS = AF_DS, DS4 = AF_DS / 4;
-    // e_t [max_kv], then the V chunk [chunk][DS]
-    extern __shared__ __align__(16) float lgs[];
+// in-order sum of lg[0..n) from 0 by the workgroup, in pieces of what
+// exact_sum_nonneg takes: the running sum is the next piece's first term
+template <int NT>
+__device__ __forceinline__ float att_sum(const float *lg, int n, ExactSumLds &xl) {
+    constexpr int MOST = NT * XSUM_M < XSUM_MAX_N ? NT * XSUM_M : XSUM_MAX_N;
+    float sum = 0.0f;
+    for (int base = 0; base < n;) {
+        const bool cont = base > 0;
+        const int cnt = min(MOST, n - base + (cont ? 1 : 0));
+        const float first = sum;
+        const float *e = lg + base - (cont ? 1 : 0);
+        const int m = xsum_run(cnt, NT), j0 = threadIdx.x * m;
+        float v[XSUM_M];
+#pragma unroll
+        for (int k = 0; k < XSUM_M; ++k) {
+            const int j = j0 + k;
+            v[k] = (k < m && j < cnt) ? (cont && j == 0 ? first : e[j]) : 0.0f;
+        }
+        sum = exact_sum_nonneg(v, cnt, NT, xl, [e, cont, first](int j) { return cont && j == 0 ? first : e[j]; });
+        base += cnt - (cont ? 1 : 0);
+    }
+    return sum;
+}
+
+// (n_kv past cap: a batched caller's position beyond its slice.) attend_decode's
+// sequence with the logits formed again, cap positions at a time.
+template <int HD, int DS, int NT>
+__device__ __forceinline__ void att_beyond_cap(const AttArgs &a, const float *q, const float *kc, const float *vc,
+                               int kv_dim, int n_kv, float *lg, float *red, const uint64_t *tab,
+                               float *out) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float mx = -INFINITY;
+    for (int t = tid; t < n_kv; t += NT)
+        mx = fmaxf(mx, att_logit<HD>(q, kc + (size_t)t * kv_dim, a.scale));
+    mx = wave_reduce(mx, -INFINITY, [](float x, float y) { return fmaxf(x, y); });
+    if (lane == 0) red[wave] = mx;
+    __syncthreads();
+    for (int w = 0; w < NT / 64; ++w) mx = fmaxf(mx, red[w]);
+    float sum = 0.0f, inv = 0.0f, acc = 0.0f;
+    for (int pass = 0; pass < 2; ++pass) {
+        for (int c0 = 0; c0 < n_kv; c0 += a.cap) {
+            const int np = min(a.cap, n_kv - c0);
+            __syncthreads();
+            for (int t = tid; t < np; t += NT)
+                lg[t] = expf_ref_tab(att_logit<HD>(q, kc + (size_t)(c0 + t) * kv_dim, a.scale) - mx, tab);
+            __syncthreads();
+            if (pass == 0) {
+                if (tid == 0)
+                    for (int t = 0; t < np; ++t) sum = sum + lg[t];
+            } else if (tid < DS) {
+                for (int t = 0; t < np; ++t) {
+                    const float w = lg[t] * inv;
+                    acc = acc + w * vc[(size_t)(c0 + t) * kv_dim + tid];
+                }
+            }
+        }
+        if (pass == 0) {
+            if (tid == 0) red[0] = __fdiv_rn(1.0f, sum);
+            __syncthreads();
+            inv = red[0];
+        }
+    }
+    if (tid < DS) out[tid] = acc;
+}
+
+// e_t summed in order from 0 by one lane, 32 read per step.
+__device__ __forceinline__ float att_sum_serial(const float *lg, int n) {
+    float sum = 0.0f;
+    int t = 0;
+    for (; t + 32 <= n; t += 32) {
+        att_f4 e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = *(const att_f4 *)(lg + t + 4 * j);
+#pragma unroll
+        for (int j = 0; j < 32; ++j) sum = sum + e[j / 4][j % 4];
+    }
+    for (; t < n; ++t) sum = sum + lg[t];
+    return sum;
+}
+
+// The logits of every position into lg, from K rows staged 64 * TILES at a
+// time in `ks` (16-byte units of row t at unit u ^ t: conflict-free reads of one
+// unit by 64 rows); returns this thread's share of their max.
+template <int HD, int NT, int TILES>
+__device__ __forceinline__ float att_logits_here(const float *q, const float *kc, int kv_dim, int n_kv,
+                                                 float scale, float *lg, float *ks) {
+    constexpr int U = HD / 4, ROWS = 64 * TILES, PER = (ROWS * U + NT - 1) / NT;
+    const int tid = threadIdx.x;
+    float mx = -INFINITY;
+    for (int t0 = 0; t0 < n_kv; t0 += ROWS) {
+        const int last = min(ROWS, n_kv - t0) - 1;
+        if (t0) __syncthreads();  // the previous rows are read
+        att_f4 r[PER];
+        // loads at clamped rows (all in flight together)
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            if (NT * k > last * U + U - 1) break;
+            const int i = tid + NT * k, t = min(i / U, last);
+            r[k] = *(const att_f4 *)(kc + (size_t)(t0 + t) * kv_dim + 4 * (i % U));
+        }
+        if (t0 == 0) att_touch<HD>((att_cptr)q);
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            if (NT * k > last * U + U - 1) break;
+            const int i = tid + NT * k, t = i / U;
+            if (t <= last) *(att_f4 *)(ks + 4 * (t * U + ((i % U) ^ (t % U)))) = r[k];
+        }
+        __syncthreads();
+        if (tid < ROWS) {
+            att_cptr qc = (att_cptr)q;
+            float dot = 0.0f;
+#pragma unroll
+            for (int u0 = 0; u0 < U; u0 += 8) {
+                att_f4 k4[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) k4[j] = *(const att_f4 *)(ks + 4 * (tid * U + ((u0 + j) ^ (tid % U))));
+#pragma unroll
+                for (int j = 0; j < 32; ++j) dot = dot + qc[4 * u0 + j] * k4[j / 4][j % 4];
+            }
+            if (tid <= last) {
+                const float l = dot * scale;
+                lg[t0 + tid] = l;
+                mx = fmaxf(mx, l);
+            }
+        }
+    }
+    return mx;
+}
+
+// WIDE: a CU to a workgroup: wave 0 folds and the producers are on the other
+// three SIMDs (wave % 4 != 0), so nothing competes with the chain for its
+// SIMD. Else DS / 64 folding waves, then the producers, several workgroups to
+// a CU.
+template <int DS, int NP, bool WIDE>
+constexpr int am_threads = WIDE ? 64 * (1 + (NP + 2) / 3 * 3 + (NP - 1) / 3) : DS + 64 * NP;
+// Positions per chunk: one 4 x 4 piece of products per producer thread, or two
+// where several workgroups share the CU (a barrier and a hand-over per 64
+// positions instead of 32).
+template <int DS, int NP, bool WIDE>
+constexpr int am_chunk = (WIDE ? 1 : 2) * 1024 * NP / DS;
+
+template <int HD, int DS, int NP, bool WIDE, int TILES>
+__global__ __launch_bounds__((am_threads<DS, NP, WIDE>)) void attend_mix(AttArgs a) {
+    constexpr int NF = DS / 64, NT = am_threads<DS, NP, WIDE>, NW = NT / 64;
+    constexpr int CH = am_chunk<DS, NP, WIDE>, HALF = CH / 2, D4 = DS / 4;
+    static_assert(!WIDE || NF == 1, "the wide form folds on one wave");
+    static_assert(NW <= 16 && CH % 32 == 0, "the workgroup's size, whole reads of a chunk");
+    // weights [cap, rounded up to 128], then 2 chunks of products or 64 * TILES K rows
+    extern __shared__ __align__(16) float dyn[];
     __shared__ ExactSumLds xl;
     __shared__ uint64_t tab[32];
     __shared__ float red[16];
     __shared__ float inv1;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int h = blockIdx.x, sd = blockIdx.y * DS;  // the head and the slice's first dimension
-    const int kv_dim = n_head_kv * HD, kvh = h / (n_head / n_head_kv);
-    const int n_kv = pos_p[0] + 1;
-    if (wave == 0) expf_ref_tab_fill(tab);
-    // the head's logits into LDS, and their max (f32::max fold: NaN
-    // ignoring, order free)
-    float mx = -INFINITY;
-    for (int t = tid; t < n_kv; t += 1024) {
-        const float l = scores[(size_t)h * max_kv + t];
-        lgs[t] = l;
-        mx = fmaxf(mx, l);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // a kv head's heads and slices on every n_head_kv-th workgroup, so that
+    // the XCD they share reads that kv head's V only
+    constexpr int SL = HD / DS;
+    const int g = blockIdx.x % a.n_head_kv, r = blockIdx.x / a.n_head_kv;
+    const int h = g * (a.n_head / a.n_head_kv) + r / SL, sd = (r % SL) * DS, s = blockIdx.y;
+    const int kv_dim = a.n_head_kv * HD, n_kv = att_n_kv(a, s);
+    const float *q = a.q + ((size_t)s * a.n_head + h) * HD;
+    const float *kc = a.kc + (size_t)s * a.seq_stride + (size_t)g * HD;
+    const float *vc = a.vc + (size_t)s * a.seq_stride + (size_t)g * HD + sd;
+    float *out = a.out + ((size_t)s * a.n_head + h) * HD + sd;
+    if (n_kv < 1 || n_kv > ATT_MAX_KV) {
+        if (tid < DS) out[tid] = __builtin_nanf("");
+        return;
     }
-    mx = wave_reduce(mx, -INFINITY, [](float a, float b) { return fmaxf(a, b); });
+    float *lg = dyn, *buf = dyn + (a.cap + 127) / 128 * 128;
+    if (wave == NW - 1) expf_ref_tab_fill(tab);
+    if (n_kv > a.cap) {
+        __syncthreads();
+        att_beyond_cap<HD, DS, NT>(a, q, kc, vc, kv_dim, n_kv, lg, red, tab, out);
+        return;
+    }
+    const int nc = (n_kv + CH - 1) / CH;
+    // a producer thread's piece of a chunk: positions 4 t4 .. 4 t4 + 3, dimensions
+    // 4 d4 .. 4 d4 + 3
+    const int pw = WIDE ? (wave >> 2) * 3 + (wave & 3) - 1 : wave - NF;
+    const bool folds = WIDE ? wave == 0 : wave < NF;
+    const bool produces = WIDE ? (wave & 3) != 0 && pw < NP : !folds;
+    const int piece = pw * 64 + lane, t4 = piece / D4, d4 = piece % D4;
+    att_f4 va[4], vb[4];
+    const float *vp = vc + 4 * d4;
+    const auto vload = [&](att_f4 (&v)[4], int t0) {  // from position t0 + 4 t4
+        const int t = t0 + 4 * t4;
+        if (t0 + CH <= n_kv) {
+            const float *p = vp + (size_t)t * kv_dim;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = *(const att_f4 *)(p + (size_t)i * kv_dim);
+        } else {  // rows past the last re-read it, unused
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = *(const att_f4 *)(vp + (size_t)min(t + i, n_kv - 1) * kv_dim);
+        }
+    };
+    // the two register sets: both halves of a chunk, or two chunks
+    constexpr int STEP = WIDE ? CH : HALF;
+    if (produces) {
+        vload(va, 0);
+        if (!WIDE || nc > 1) vload(vb, STEP);
+    }
+    // the logits and their max (f32::max fold: NaN ignoring, order free)
+    float mx = -INFINITY;
+    if (n_kv <= a.fuse) {
+        mx = att_logits_here<HD, NT, TILES>(q, kc, kv_dim, n_kv, a.scale, lg, buf);
+    } else {
+        const float *sc = a.scores + ((size_t)s * a.n_head + h) * a.cap;
+        for (int t = tid; t < n_kv; t += NT) {
+            const float l = sc[t];
+            lg[t] = l;
+            mx = fmaxf(mx, l);
+        }
+    }
+    mx = wave_reduce(mx, -INFINITY, [](float x, float y) { return fmaxf(x, y); });
     if (lane == 0) red[wave] = mx;
     __syncthreads();
     mx = -INFINITY;
-    for (int w = 0; w < 16; ++w) mx = fmaxf(mx, red[w]);
-    for (int t = tid; t < n_kv; t += 1024) lgs[t] = expf_ref_tab(lgs[t] - mx, tab);
-    __syncthreads();
-    // their sum in order from 0, by the workgroup
-    {
-        const int m = xsum_run(n_kv, 1024), j0 = tid * m;
-        float v[XSUM_M];
 #pragma unroll
-        for (int k = 0; k < XSUM_M; ++k) v[k] = (k < m && j0 + k < n_kv) ? lgs[j0 + k] : 0.0f;
-        const float *e = lgs;
-        const float sum = exact_sum_nonneg(v, n_kv, 1024, xl, [e](int j) { return e[j]; });
+    for (int w = 0; w < NW; ++w) mx = fmaxf(mx, red[w]);
+    for (int t = tid; t < n_kv; t += NT) lg[t] = expf_ref_tab(lg[t] - mx, tab);
+    __syncthreads();
+    if (n_kv <= ATT_SERIAL) {
+        if (tid == 0) inv1 = __fdiv_rn(1.0f, att_sum_serial(lg, n_kv));
+    } else {
+        const float sum = att_sum<NT>(lg, n_kv, xl);
         if (tid == 0) inv1 = __fdiv_rn(1.0f, sum);
     }
     __syncthreads();
-    // the weighted V sum, one thread per dimension of this slice, in
-    // position order, from V rows staged in LDS a chunk at a time: the next
-    // chunk's loads (all threads, into registers) are in flight while this
-    // one is folded
-    float *vst = lgs + max_kv;                    // [chunk][DS]
-    const int units = chunk * DS4;                // float4s per chunk
-    att_f4 reg[AF_PER];
-    // every load unconditional, at a clamped row (a conditional load makes
-    // the compiler wait for each one before issuing the next); the extra
-    // ones re-read a row of the chunk and are never stored
-    const auto stage_load = [&](int c0) {
-        const int last = min(chunk, n_kv - c0) - 1;
-#pragma unroll
-        for (int k = 0; k < AF_PER; ++k) {
-            const int i = tid + 1024 * k;
-            const int t = min(i / DS4, last), d4 = i % DS4;
-            reg[k] = *(const att_f4 *)(vc + (size_t)(c0 + t) * kv_dim + (size_t)kvh * HD + sd + 4 * d4);
-        }
-    };
-    const auto stage_store = [&](int c0) {
-        const int np = min(chunk, n_kv - c0);
-#pragma unroll
-        for (int k = 0; k < AF_PER; ++k) {
-            const int i = tid + 1024 * k;
-            if (i < units && i / DS4 < np) *(att_f4 *)(vst + 4 * i) = reg[k];
-        }
-    };
-    const bool folder = tid < DS;
     const float inv = inv1;
-    float acc = 0.0f;
-    stage_load(0);
-    for (int c0 = 0; c0 < n_kv; c0 += chunk) {
-        stage_store(c0);
-        __syncthreads();
-        if (c0 + chunk < n_kv) stage_load(c0 + chunk);
-        if (folder) {
-            const int np = min(chunk, n_kv - c0);
-            const float *vr = vst + tid;
-            int t = 0;
-            for (; t + 8 <= np; t += 8) {
-                // the 8 values and their 8 weights read together, then the
-                // ordered adds (lgs + c0 + t is 16-byte aligned: c0 and t are
-                // multiples of 8)
-                float vv[8];
+
+    // products of chunk c into its buffer; positions past the last add +0.0,
+    // which leaves every sum as it is (a sum from +0.0 is never -0.0)
+    const auto produce = [&](const att_f4 (&v)[4], int c, int half) {
+        const int t0 = c * CH + half * HALF, t = t0 + 4 * t4;
+        const att_f4 e = *(const att_f4 *)(lg + t);
+        att_f4 p[4];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) vv[j] = vr[(size_t)(t + j) * DS];
-                const float4 e0 = *(const float4 *)(lgs + c0 + t), e1 = *(const float4 *)(lgs + c0 + t + 4);
-                const float ee[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
+        for (int i = 0; i < 4; ++i) {
+            const float w = e[i] * inv;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float w = ee[j] * inv;
-                    acc = acc + w * vv[j];
-                }
-            }
-            for (; t < np; ++t) {
-                const float w = lgs[c0 + t] * inv;
-                acc = acc + w * vr[(size_t)t * DS];
+            for (int j = 0; j < 4; ++j) p[j][i] = w * v[i][j];
+        }
+        if (t0 + CH > n_kv) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) p[j][i] = t + i < n_kv ? p[j][i] : 0.0f;
+        }
+        // dimension 4 d4 + j in slot j * D4 + d4: a wave's stores are contiguous
+        float *dst = buf + (c & 1) * (CH * DS) + half * (HALF * DS) + t4 * DS * 4 + d4 * 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *(att_f4 *)(dst + j * D4 * 4) = p[j];
+    };
+    // Chunk c is folded between barriers c and c + 1, while chunk c + 1 goes
+    // into the other buffer. The folding and the producing waves have loops of
+    // their own (a shared loop's register merges would wait for the loads in
+    // flight).
+    if (folds) {
+        __builtin_amdgcn_s_setprio(3);
+        float acc = 0.0f;
+        for (int c = 0; c < nc; ++c) {
+            __syncthreads();
+            const float *src = buf + (c & 1) * (CH * DS) + tid * 4;
+            // 32 products ahead of the 32 being added
+            att_f4 p[2][8];
+            const auto read = [&](int k) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) p[k & 1][i] = *(const att_f4 *)(src + (8 * k + i) * DS * 4);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            read(0);
+#pragma unroll
+            for (int k = 0; k < CH / 32; ++k) {
+                if (k + 1 < CH / 32) read(k + 1);
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc = acc + p[k & 1][i][e];
             }
         }
-        __syncthreads();  // the chunk is read before the next one is stored
+        out[(tid % D4) * 4 + tid / D4] = acc;
+    } else if (produces) {
+        if constexpr (WIDE) {
+            produce(va, 0, 0);
+            if (nc > 2) vload(va, 2 * CH);
+            for (int c = 0; c < nc; c += 2) {
+                __syncthreads();
+                if (c + 1 >= nc) break;
+                produce(vb, c + 1, 0);
+                if (c + 3 < nc) vload(vb, (c + 3) * CH);
+                __syncthreads();
+                if (c + 2 >= nc) break;
+                produce(va, c + 2, 0);
+                if (c + 4 < nc) vload(va, (c + 4) * CH);
+            }
+        } else {
+            for (int c = 0; c < nc; ++c) {
+                if (c) __syncthreads();
+                produce(va, c, 0);
+                if (c + 1 < nc) vload(va, (c + 1) * CH);
+                produce(vb, c, 1);
+                if (c + 1 < nc) vload(vb, (c + 1) * CH + HALF);
+            }
+            __syncthreads();
+        }
+    } else {
+        for (int c = 0; c < nc; ++c) __syncthreads();
     }
-    if (folder) out[(size_t)h * HD + sd + tid] = acc;
 }
 
 }  // namespace
@@ -687,58 +929,84 @@ int launch_attend_fused(const float *q, const float *k, const float *v, const fl
 }
 
 namespace {
-size_t g_split_lds = 0;  // the dynamic LDS attend_finish may use (raised by prepare)
-
-// V positions per LDS chunk: what the e_t rows leave of 152 KB, at most
-// AF_PER float4s per thread, a multiple of 16 (0: does not fit)
-int split_chunk(int n_head, int n_head_kv, int max_kv) {
-    (void)n_head;
-    (void)n_head_kv;
-    const long room = 152L * 1024 - (long)max_kv * 4 - 8 * 1024;
-    long c = room / (AF_DS * 4);
-    c = std::min<long>(c, (long)AF_PER * 1024 / (AF_DS / 4));
-    c -= c % 16;
-    return c >= 16 ? (int)c : 0;
+size_t split_lds(int cap, int hd, int ds, int chunk, int tiles) {
+    return (size_t)(cap + 127) / 128 * 128 * 4 + std::max(2 * chunk * ds * 4, tiles * 64 * hd * 4);
 }
-size_t split_lds(int n_head, int n_head_kv, int max_kv) {
-    return (size_t)max_kv * 4 + (size_t)split_chunk(n_head, n_head_kv, max_kv) * AF_DS * 4;
+
+template <int HD, int DS, int NP, bool WIDE, int TILES>
+int launch_mix(const AttArgs &a, int nseq, hipStream_t st) {
+    constexpr int CH = am_chunk<DS, NP, WIDE>;
+    // the largest cache's dynamic LDS, allowed once per kernel
+    static const hipError_t ok = hipFuncSetAttribute((const void *)attend_mix<HD, DS, NP, WIDE, TILES>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     (int)split_lds(ATT_MAX_KV, HD, DS, CH, TILES));
+    if (ok != hipSuccess) return -1;
+    hipLaunchKernelGGL((attend_mix<HD, DS, NP, WIDE, TILES>), dim3(a.n_head * (HD / DS), nseq),
+                       dim3(am_threads<DS, NP, WIDE>), split_lds(a.cap, HD, DS, CH, TILES), st, a);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 }  // namespace
 
 bool attend_split_fits(int n_head, int n_head_kv, int hd, int max_kv) {
-    if (hd != ATT_HD || n_head_kv <= 0 || n_head % n_head_kv || n_head % 2 || max_kv <= 0) return false;
-    const int group = n_head / n_head_kv;
-    return group <= AL_MAX_GROUP && split_chunk(n_head, n_head_kv, max_kv) > 0;
+    return (hd == 64 || hd == 128) && n_head_kv > 0 && n_head_kv <= 65535 && n_head > 0 &&
+           n_head % n_head_kv == 0 && n_head / n_head_kv <= AS_MAX_GROUP && max_kv > 0 &&
+           max_kv <= ATT_MAX_KV;
 }
 
-int attend_split_prepare(int n_head, int n_head_kv, int hd, int max_kv) {
-    if (!attend_split_fits(n_head, n_head_kv, hd, max_kv)) return -1;
-    const size_t lds = split_lds(n_head, n_head_kv, max_kv);
-    if (lds <= g_split_lds) return 0;
-    if (hipFuncSetAttribute((const void *)attend_finish, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds) != hipSuccess)
-        return -1;
-    g_split_lds = lds;
-    return 0;
-}
+size_t attend_split_scores(int n_head, int cap, int nseq) { return (size_t)nseq * n_head * cap; }
 
 int launch_attend_split(const float *q, const float *kc, const float *vc, const int32_t *pos,
-                        int n_head, int n_head_kv, int hd, float scale, int max_kv, float *scores,
-                        int8_t *oq, float *od, float *out, hipStream_t st) {
-    if (!attend_split_fits(n_head, n_head_kv, hd, max_kv) || !out) return -1;
-    const size_t lds = split_lds(n_head, n_head_kv, max_kv);
-    if (lds > g_split_lds) return -1;  // attend_split_prepare first
-    const int chunk = split_chunk(n_head, n_head_kv, max_kv);
-    // 256 workgroups (a multiple of n_head_kv), each fixed to one kv head
-    const int grid = (256 / n_head_kv) * n_head_kv;
-    if (grid <= 0) return -1;
-    hipLaunchKernelGGL(attend_logits, dim3(grid), dim3(256), 0, st, q, kc, pos, n_head, n_head_kv,
-                       scale, scores, max_kv);
-    hipLaunchKernelGGL(attend_finish, dim3(n_head, AF_SL), dim3(1024), lds, st, scores, vc, pos,
-                       n_head, n_head_kv, max_kv, chunk, out);
+                        int n_head, int n_head_kv, int hd, float scale, int cap, float *scores,
+                        float *out, hipStream_t st, int nseq, int n_kv_fixed, int pos_stride,
+                        size_t cache_seq_stride, int expect) {
+    if (!attend_split_fits(n_head, n_head_kv, hd, cap) || nseq <= 0 || nseq > 65535) return -1;
+    if (expect <= 0 || expect > cap) expect = cap;
+    AttArgs a{};
+    a.q = q;
+    a.kc = kc;
+    a.vc = vc;
+    a.pos_p = pos;
+    a.scores = scores;
+    a.out = out;
+    a.seq_stride = cache_seq_stride;
+    a.pos_stride = pos_stride;
+    a.n_kv_fixed = n_kv_fixed;
+    a.n_head = n_head;
+    a.n_head_kv = n_head_kv;
+    a.cap = cap;
+    a.scale = scale;
+    const int heads = nseq * n_head;
+    // us per call with the Q8_K behind it, 32 query / 4 kv heads of 128
+    // (attend_decode alone, then this): 1 sequence of 250 positions 15.2, 13.2;
+    // 1000: 49, 16.8; 4100: 278, 34.5; 8192: 544, 56; 13 of up to 1000: 88, 29;
+    // 16 of up to 2000: 185, 49; of up to 40: 10.5, 8.9.
+    if (expect <= 256) {
+        // short caches: one launch of small workgroups that form the logits
+        // themselves (at 300 positions the second launch already pays)
+        a.fuse = cap;
+        if (hd == 64) return launch_mix<64, 64, 4, false, 2>(a, nseq, st);
+        return heads <= 128 ? launch_mix<128, 64, 4, false, 2>(a, nseq, st)
+                            : launch_mix<128, 128, 4, false, 1>(a, nseq, st);
+    }
+    a.fuse = 64;
+    const int blocks = (expect + AS_POS - 1) / AS_POS;
+    const int share = 2048 / (n_head_kv * nseq);
+    a.grid_x = blocks < share ? blocks : share > 0 ? share : 1;
+    const dim3 grid(a.grid_x, n_head_kv, nseq), block(64 * (n_head / n_head_kv));
+    if (hd == 128) hipLaunchKernelGGL(attend_scores<128>, grid, block, 0, st, a);
+    else hipLaunchKernelGGL(attend_scores<64>, grid, block, 0, st, a);
     if (hipGetLastError() != hipSuccess) return -1;
-    // oq null: the caller takes the f32 output (launch_q6k_mv_f32x)
-    return oq ? launch_q8k_quantize(out, oq, od, nullptr, n_head / 2, st) : 0;
+    // a CU to a workgroup while every one finds its own (1..4 sequences of
+    // 1000: 16.8-18.3 us, 17.2-18.7 with the small workgroups); then small
+    // workgroups on 64 dimensions up to one per CU and dimension half (8 of
+    // 500: 16.9, 18.9 with all 128 dimensions), then on all (13 of 1000: 28.9,
+    // 36 with 64)
+    if (hd == 64)
+        return heads <= 128 ? launch_mix<64, 64, 8, true, 1>(a, nseq, st)
+                            : launch_mix<64, 64, 4, false, 1>(a, nseq, st);
+    if (heads <= 128) return launch_mix<128, 64, 8, true, 1>(a, nseq, st);
+    return heads <= 256 ? launch_mix<128, 64, 4, false, 1>(a, nseq, st)
+                        : launch_mix<128, 128, 4, false, 1>(a, nseq, st);
 }
 
 int launch_attend_decode(const float *q, const float *kc, const float *vc, const int32_t *pos,

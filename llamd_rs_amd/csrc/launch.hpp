@@ -212,17 +212,20 @@ int launch_attend_fused(const float *q, const float *k, const float *v, const fl
 // (pf0 / pf1: n0 + n1 extra workgroups read b0 (b1) bytes each from pf0 + i * b0
 // (pf1 + i * b1) into the L2 of XCD i % 8, where workgroup i of the later launch that
 // reads them runs; needs n_head / 2 and n0 to be multiples of 8, else skipped)
-// Attention over long contexts in two launches (after launch_qk_norm_rope_store):
-// logits spread over 256 workgroups, then the softmax (exact in-order sum)
-// and the in-order weighted V sum (two workgroups per head) into out
-// [n_head * hd], and its Q8_K; the bits of launch_attend_fused. scores:
-// [n_head][max_kv] floats.
+// Attention spread over the GPU (q normed and rotated, K and V in the cache):
+// the logits by blocks of positions, then the softmax (exact in-order sum) and
+// the in-order weighted V sum per head, into out [nseq][n_head * hd]; the bits
+// of launch_attend_decode. cap: positions that scores (attend_split_scores
+// floats) and the LDS hold per head; a sequence that has more is still
+// attended to, slowly. expect: the most positions a sequence is expected to
+// have (0: cap), which only decides how the work is split. Sequences as in
+// launch_attend_decode.
 bool attend_split_fits(int n_head, int n_head_kv, int hd, int max_kv);
-// raises attend_finish's dynamic LDS limit for max_kv positions (outside graph capture)
-int attend_split_prepare(int n_head, int n_head_kv, int hd, int max_kv);
+size_t attend_split_scores(int n_head, int cap, int nseq);
 int launch_attend_split(const float *q, const float *kc, const float *vc, const int32_t *pos,
-                        int n_head, int n_head_kv, int hd, float scale, int max_kv, float *scores,
-                        int8_t *oq, float *od, float *out, hipStream_t st);
+                        int n_head, int n_head_kv, int hd, float scale, int cap, float *scores,
+                        float *out, hipStream_t st, int nseq = 1, int n_kv_fixed = 0,
+                        int pos_stride = 0, size_t cache_seq_stride = 0, int expect = 0);
 // nseq sequences: n_kv = pos[s * pos_stride] + 1 (pos null: n_kv_fixed); q, out
 // [nseq][n_head * hd]; sequence s's cache starts cache_seq_stride floats after s-1's.
 int launch_attend_decode(const float *q, const float *kc, const float *vc, const int32_t *pos,

@@ -117,7 +117,7 @@ bool enqueue_step(Model *m, hipStream_t st, bool long_ctx) {
                                                    m->eps, l.kc, l.vc, st);
             rc |= llamd::launch_attend_split(m->q, l.kc, l.vc, m->tokpos + 1, m->n_head,
                                              m->n_head_kv, m->hd, m->scale, m->max_kv, m->scores,
-                                             nullptr, nullptr, m->attn, st);
+                                             m->attn, st);
         } else if (m->fused_attn) {
             // with the O projection's weight tiles and the MoE router's
             // rows read into L2 alongside, each on the XCD of the workgroup
@@ -249,7 +249,7 @@ void *llamd_hip_model_create(void *g, int max_kv) {
     m->long_from = llamd::g_tune_model_long_from;
     m->split_attn = m->long_from >= 0 && m->long_from < max_kv &&
                     (int)(n_head * hd) / 256 <= 16 &&  // the f32-input O matvec (launch_q6k_mv_f32x)
-                    llamd::attend_split_prepare((int)n_head, (int)n_head_kv, (int)hd, max_kv) == 0;
+                    llamd::attend_split_fits((int)n_head, (int)n_head_kv, (int)hd, max_kv);
     m->eps = eps;
     m->rope_base = base;
     m->scale = 1.0f / sqrtf((float)hd);  // attention.rs:95
@@ -350,7 +350,7 @@ void *llamd_hip_model_create(void *g, int max_kv) {
     m->tokpos = (int32_t *)dalloc(*m, 16);
     m->next = (int32_t *)dalloc(*m, 16);
     if (m->split_attn) {
-        m->scores = dalloc(*m, (size_t)m->n_head * max_kv * 4);
+        m->scores = dalloc(*m, llamd::attend_split_scores(m->n_head, max_kv, 1) * 4);
         if (!m->scores) m->split_attn = false;
     }
     if (hipHostMalloc((void **)&m->stage, 64, hipHostMallocDefault) != hipSuccess) m->stage = nullptr;
