@@ -121,9 +121,8 @@ __global__ __launch_bounds__(256) void act_unbias(const uint32_t *q, uint32_t fl
 }
 
 // Natural-layout quants and scales of n_act tokens -> the token-chunked
-// operand layout of q6k_mv_batched (q8k_wave.hpp): block b of chunk k is 4 KiB
-// at (k * blocks + b) * 4096, class plane c = e % 8 at c * 512, token n of the
-// chunk at n * 32, byte e / 8. Token slots past n_act are zero.
+// operand layout of q6k_mv_batched (chunk_byte, q8k_wave.hpp). Token slots past
+// n_act are zero.
 __global__ __launch_bounds__(256) void act_to_chunks(const uint8_t *q, const float *d, uint8_t flip,
                                                      int n_act, int blocks, uint8_t *cq, float *cd,
                                                      size_t n_bytes, unsigned nblk) {
@@ -132,7 +131,9 @@ __global__ __launch_bounds__(256) void act_to_chunks(const uint8_t *q, const flo
         const size_t kb = D >> 12;  // chunk * blocks + block
         const int w = (int)(D & 4095);
         const int k = (int)(kb / blocks), b = (int)(kb - (size_t)k * blocks);
-        const int c = w >> 9, tn = (w & 511) >> 5, m = w & 31;
+        // chunk_byte's inverse
+        const int unit = (w & 1023) >> 4, tn = unit & 15;
+        const int c = 2 * (w >> 10) + ((w >> 3) & 1), m = 8 * (unit >> 4) + (w & 7);
         const int t = 16 * k + tn, e = 8 * m + c;
         cq[D] = t < n_act ? (uint8_t)(q[((size_t)t * blocks + b) * QK_K + e] ^ flip) : (uint8_t)0;
         if (w < 16) {

@@ -10,6 +10,13 @@
 
 namespace llamd {
 
+// The byte of weight e of token n within its (chunk, block)'s 4 KiB of the
+// token-chunked activations (q8k_wave.hpp).
+__host__ __device__ constexpr int chunk_byte(int e, int n) {
+    const int c = e & 7, m = e >> 3;
+    return (c >> 1) * 1024 + ((m >> 3) * 16 + n) * 16 + (c & 1) * 8 + (m & 7);
+}
+
 // Tuning overrides (0 = automatic); set through llamd_hip_tune.
 extern int g_tune_batched_twin;
 extern int g_tune_fast_lds;  // LLAMD_HIP_REDUCTION LM head: the chunk's quants staged in LDS
@@ -105,7 +112,8 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
                           const float *act_d, float *y, int ldy, int rows, int blocks,
                           int n_groups, int max_chunks, hipStream_t st, float *amax_v = nullptr,
                           int *amax_i = nullptr, bool group_tables = false,
-                          const void *w2 = nullptr, float *y2 = nullptr, bool fast = false);
+                          const void *w2 = nullptr, float *y2 = nullptr, bool fast = false,
+                          bool few = false);
 // Grouped (grp_expert set): sub_start holds 2 * (n_groups + 1) entries, the
 // chunk prefix sub_start[0..n_groups] and the twin prefix after it
 // (launch_moe_group's layout); group_tables: the GroupItem records follow
@@ -114,6 +122,8 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
 // the same activations, in the same launch. fast: the REDUCTION-tolerance
 // kernels (one float accumulator per output instead of the reference's eight
 // class sums; outputs within REDUCTION of dot_q6k_q8k, not bit-identical).
+// few: exact grouped calls (with group_tables) that leave most groups a token
+// or two.
 // Up to three matrices with their own row counts (Q, K, V) against the same
 // nseq token-chunked activations, one launch: y[i] [nseq][rows[i]].
 int launch_q6k_mv_batched_x3(const void *const w[3], float *const y[3], const int rows[3], int n_mat,

@@ -438,8 +438,7 @@ struct BatchParams {
 
 // The work item of this wave and the parameters it runs with: the second
 // matrix's items are the first's, offset by items_per_mat.
-__device__ __forceinline__ int batch_item(const BatchParams &p, BatchParams &q) {
-    int item = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
+__device__ __forceinline__ int batch_item(const BatchParams &p, BatchParams &q, int item) {
     q = p;
     if (p.n_segs > 0) {
         // the item's segment, chosen with scalar selects
@@ -459,6 +458,9 @@ __device__ __forceinline__ int batch_item(const BatchParams &p, BatchParams &q) 
         q.y = p.y2;
     }
     return item;
+}
+__device__ __forceinline__ int batch_item(const BatchParams &p, BatchParams &q) {
+    return batch_item(p, q, (int)blockIdx.x * 4 + (threadIdx.x >> 6));
 }
 
 typedef short s16x2 __attribute__((ext_vector_type(2)));
@@ -507,6 +509,111 @@ __device__ __forceinline__ void fold_digits(uint64_t codes, const FoldScales &f,
 }
 
 
+// The outputs of batched_tile's sums: y, and the tile's arg-max candidates.
+template <int NC>
+__device__ __forceinline__ void batched_store(const BatchParams &p, const float (&sums)[NC][8][4], int lane,
+                                              int t, int st0, int cnt, int start) {
+    const int n = lane & 15, s = lane >> 4;
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const int tok = 16 * (st0 + u) + n;  // this lane's token (B operand / output column)
+        const bool tok_ok = tok < cnt;       // slots past the last token hold no data;
+                                             // their columns are never stored
+        float bv = -INFINITY;  // arg-max candidate of this lane's rows (lowest row on ties)
+        int bi = 0x7FFFFFFF;
+        if (tok_ok) {
+            const int pos = start + tok;
+            const int orow = p.pair_out ? p.pair_out[pos] : pos;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = t * TILE_ROWS + 4 * s + v;
+                if (row < p.rows) {
+                    float tot = -0.0f;
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) tot = tot + sums[u][c][v];
+                    p.y[(size_t)orow * p.ldy + row] = tot;
+                    if (!isnan(tot)) argmax_step(bv, bi, tot, row);
+                }
+            }
+        }
+        if (p.amax_v) {
+            // combine the 4 lanes (s = 0..3) of each token: lanes n, n+16, n+32, n+48
+            argmax_step(bv, bi, __shfl_xor(bv, 16, WAVE), __shfl_xor(bi, 16, WAVE));
+            argmax_step(bv, bi, __shfl_xor(bv, 32, WAVE), __shfl_xor(bi, 32, WAVE));
+            if (s == 0 && tok_ok) {
+                p.amax_v[(size_t)tok * p.tiles + t] = bv;
+                p.amax_i[(size_t)tok * p.tiles + t] = bi;
+            }
+        }
+    }
+}
+
+// One block of a tile against NC chunks whose planes lie in LDS at aq (this
+// lane's 16 bytes of the first plane; chunks CHUNK_BLOCK_BYTES apart): the
+// integer dots of all 8 classes and the reference's ordered sums.
+struct TileRegs {
+    uint4 q0, q1, q2;
+    uint32_t scw;
+    uint2 dw;
+};
+__device__ __forceinline__ void tile_load(TileRegs &r, const uint8_t *sg, int lane) {
+    r.q0 = *(const uint4 *)(sg + 16 * lane);
+    r.q1 = *(const uint4 *)(sg + SEG_PART + 16 * lane);
+    r.q2 = *(const uint4 *)(sg + 2 * SEG_PART + 16 * lane);
+    r.scw = *(const uint32_t *)(sg + SEG_SC + 4 * lane);
+    r.dw = *(const uint2 *)(sg + SEG_D + 8 * (lane >> 4));  // f16 d of rows 4s..4s+3
+}
+
+__device__ __forceinline__ long plane_half(v4i v, int h) {
+    return (long)((uint64_t)(uint32_t)v[2 * h] | ((uint64_t)(uint32_t)v[2 * h + 1] << 32));
+}
+
+template <int NC>
+__device__ __forceinline__ void tile_block(const TileRegs &r, const float (&adb)[NC], const int8_t *aq,
+                                           float (&sums)[NC][8][4]) {
+    const uint32_t nib[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
+    const uint32_t hb[4] = {r.q2.x, r.q2.y, r.q2.z, r.q2.w};
+    const FoldScales fs = fold_scales(r.scw);
+    const float d4[4] = {f16_bits_to_f32((uint16_t)(r.dw.x & 0xFFFF)), f16_bits_to_f32((uint16_t)(r.dw.x >> 16)),
+                         f16_bits_to_f32((uint16_t)(r.dw.y & 0xFFFF)), f16_bits_to_f32((uint16_t)(r.dw.y >> 16))};
+    float dd[NC][4];
+#pragma unroll
+    for (int u = 0; u < NC; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dd[u][v] = d4[v] * adb[u];
+    const v4i zero = {0, 0, 0, 0};
+    v4i act[2][NC], dh[2][NC], dl[2][NC];
+    const auto read = [&](int P) {
+#pragma unroll
+        for (int u = 0; u < NC; ++u) act[P & 1][u] = *(const v4i *)(aq + u * CHUNK_BLOCK_BYTES + 1024 * P);
+    };
+    // class c's MFMAs are issued before class c - 1's results are used
+    const auto dots = [&](int c) {
+        long a_lo, a_hi;
+        fold_digits((uint64_t)unpack_codes(nib, hb, c), fs, a_lo, a_hi);
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const long av = plane_half(act[(c >> 1) & 1][u], c & 1);
+            dh[c & 1][u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, av, zero, 0, 0, 0);
+            dl[c & 1][u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, av, zero, 0, 0, 0);
+        }
+    };
+    read(0);
+    dots(0);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        if ((c & 1) == 0 && c + 2 < 8) read((c >> 1) + 1);
+        if (c + 1 < 8) dots(c + 1);
+#pragma unroll
+        for (int u = 0; u < NC; ++u)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int aux = dh[c & 1][u][v] * 256 + dl[c & 1][u][v];
+                sums[u][c][v] = sums[u][c][v] + dd[u][v] * (float)aux;
+            }
+    }
+}
+
 // The work of one wave on one 16-row tile t of expert `expert`'s weights
 // against NC consecutive 16-token chunks sub0.. of the token-chunked
 // activations (local chunk numbers st0.. inside the group of `cnt` pairs
@@ -520,7 +627,7 @@ __device__ __forceinline__ void batched_tile(const BatchParams &p, int lane, int
     const int n = lane & 15, s = lane >> 4;
     const uint8_t *seg = p.w + (size_t)expert * p.expert_stride + (size_t)t * p.blocks * SEG_BYTES;
     const size_t chunk_q = (size_t)p.blocks * CHUNK_BLOCK_BYTES, chunk_d = (size_t)p.blocks * CHUNK_TOKENS;
-    const int8_t *aq = p.act_q + (size_t)sub0 * chunk_q + n * 32 + 8 * s;
+    const int8_t *aq = p.act_q + (size_t)sub0 * chunk_q + 16 * lane;
     const float *ad = p.act_d + (size_t)sub0 * chunk_d + n;
 
     float sums[NC][8][4];
@@ -560,7 +667,8 @@ __device__ __forceinline__ void batched_tile(const BatchParams &p, int lane, int
     auto aload = [&](int b, int c) {
 #pragma unroll
         for (int u = 0; u < NC; ++u)
-            act[c % BQ][u] = *(const long *)(aq + u * chunk_q + (size_t)min(b, last) * CHUNK_BLOCK_BYTES + 512 * c);
+            act[c % BQ][u] = *(const long *)(aq + u * chunk_q + (size_t)min(b, last) * CHUNK_BLOCK_BYTES +
+                                             1024 * (c >> 1) + 8 * (c & 1));
     };
     auto compute = [&](const Regs &r, int b) {
         const uint32_t nib[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
@@ -636,38 +744,7 @@ __device__ __forceinline__ void batched_tile(const BatchParams &p, int lane, int
             compute(r, b);
         }
     }
-#pragma unroll
-    for (int u = 0; u < NC; ++u) {
-        const int tok = 16 * (st0 + u) + n;  // this lane's token (B operand / output column)
-        const bool tok_ok = tok < cnt;       // slots past the last token hold no data;
-                                             // their columns are never stored
-        float bv = -INFINITY;  // arg-max candidate of this lane's rows (lowest row on ties)
-        int bi = 0x7FFFFFFF;
-        if (tok_ok) {
-            const int pos = start + tok;
-            const int orow = p.pair_out ? p.pair_out[pos] : pos;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = t * TILE_ROWS + 4 * s + v;
-                if (row < p.rows) {
-                    float tot = -0.0f;
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) tot = tot + sums[u][c][v];
-                    p.y[(size_t)orow * p.ldy + row] = tot;
-                    if (!isnan(tot)) argmax_step(bv, bi, tot, row);
-                }
-            }
-        }
-        if (p.amax_v) {
-            // combine the 4 lanes (s = 0..3) of each token: lanes n, n+16, n+32, n+48
-            argmax_step(bv, bi, __shfl_xor(bv, 16, WAVE), __shfl_xor(bi, 16, WAVE));
-            argmax_step(bv, bi, __shfl_xor(bv, 32, WAVE), __shfl_xor(bi, 32, WAVE));
-            if (s == 0 && tok_ok) {
-                p.amax_v[(size_t)tok * p.tiles + t] = bv;
-                p.amax_i[(size_t)tok * p.tiles + t] = bi;
-            }
-        }
-    }
+    batched_store<NC>(p, sums, lane, t, st0, cnt, start);
 }
 
 // One wave per (group, 16-token chunk, 16-row tile). The chunk index is the
@@ -774,44 +851,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // The dynamic LDS of the LDSA kernels below.
 extern __shared__ uint4 g_act_lds[];
 
-// Activation planes in LDS are stored with a swizzle: in each 512-byte plane
-// (16 tokens x 32 bytes), the two 16-byte halves of token n's row are swapped
-// when bit 2 of n is set. The MFMA lane (token n, quarter s) reads 8 bytes at
-// 32 n + 8 s; without the swap, tokens n and n + 4 hit the same banks and a
-// plane read has 4-way bank conflicts, with it 2-way at most (the 16-byte
-// unit of the global-to-LDS copies allows no finer move).
-__device__ __forceinline__ int act_lds_byte(int n, int s) {
-    return 32 * n + 16 * ((s >> 1) ^ ((n >> 2) & 1)) + 8 * (s & 1);
-}
-// The global 16-byte unit (offset within the chunk's block) that LDS unit
-// `slot` of the same block holds: the swap is its own inverse.
-__device__ __forceinline__ int act_lds_src(int slot) {
-    const int n = (slot >> 1) & 15;
-    return 16 * (slot ^ ((n >> 2) & 1));
+// LDSA: the chunk's quants are read from g_act_lds (same layout).
+// The digit operands of the 64-deep MFMA of classes 2 P and 2 P + 1.
+__device__ __forceinline__ void fold_pair(const uint32_t nib[8], const uint32_t hb[4], int P,
+                                          const FoldScales &fs, v4i &lo, v4i &hi) {
+    long l[2], h[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fold_digits((uint64_t)unpack_codes(nib, hb, 2 * P + i), fs, l[i], h[i]);
+    lo = v4i{(int)l[0], (int)(l[0] >> 32), (int)l[1], (int)(l[1] >> 32)};
+    hi = v4i{(int)h[0], (int)(h[0] >> 32), (int)h[1], (int)(h[1] >> 32)};
 }
 
-// LDSA: the chunk's quants are read from g_act_lds (same layout).
 template <int NC, bool LDSA = false>
 __device__ __forceinline__ void fast_tile_range(const BatchParams &p, int lane, int t, int sub0,
                                                 int expert, int b0, int b1, float acc[2][4]) {
     const int n = lane & 15, s = lane >> 4;
     const uint8_t *seg = p.w + (size_t)expert * p.expert_stride + (size_t)t * p.blocks * SEG_BYTES;
     const size_t chunk_q = (size_t)p.blocks * CHUNK_BLOCK_BYTES, chunk_d = (size_t)p.blocks * CHUNK_TOKENS;
-    const int8_t *aq = LDSA ? (const int8_t *)g_act_lds + act_lds_byte(n, s)
-                            : p.act_q + (size_t)sub0 * chunk_q + n * 32 + 8 * s;
+    const int8_t *aq = LDSA ? (const int8_t *)g_act_lds + 16 * lane
+                            : p.act_q + (size_t)sub0 * chunk_q + 16 * lane;
     const float *ad = p.act_d + (size_t)sub0 * chunk_d + n;
-    // class planes two classes ahead of their MFMAs, across blocks (past the
+    // planes of two classes one ahead of their MFMAs, across blocks (past the
     // range's last block the loads re-read it, unused)
-    constexpr int BQ = 2;
     const int last = b1 - 1;
-    long act[BQ][NC];
-    auto aload = [&](int b, int c) {
+    v4i act[2][NC];
+    auto aload = [&](int b, int P) {
 #pragma unroll
         for (int u = 0; u < NC; ++u)
-            act[c % BQ][u] = *(const long *)(aq + u * chunk_q + (size_t)min(b, last) * CHUNK_BLOCK_BYTES + 512 * c);
+            act[P % 2][u] = *(const v4i *)(aq + u * chunk_q + (size_t)min(b, last) * CHUNK_BLOCK_BYTES + 1024 * P);
     };
-#pragma unroll
-    for (int c = 0; c < BQ; ++c) aload(b0, c);
+    aload(b0, 0);
     struct W {
         uint4 q0, q1, q2;
         uint32_t scw;
@@ -837,15 +906,15 @@ __device__ __forceinline__ void fast_tile_range(const BatchParams &p, int lane, 
 #pragma unroll
         for (int u = 0; u < NC; ++u) ah[u] = al[u] = zero;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            long a_lo, a_hi;
-            fold_digits((uint64_t)unpack_codes(nib, hb, c), fs, a_lo, a_hi);
+        for (int P = 0; P < 4; ++P) {
+            aload(P + 1 < 4 ? b : b + 1, (P + 1) % 4);
+            v4i a_lo, a_hi;
+            fold_pair(nib, hb, P, fs, a_lo, a_hi);
 #pragma unroll
             for (int u = 0; u < NC; ++u) {
-                ah[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, act[c % BQ][u], ah[u], 0, 0, 0);
-                al[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, act[c % BQ][u], al[u], 0, 0, 0);
+                ah[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_hi, act[P % 2][u], ah[u], 0, 0, 0);
+                al[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_lo, act[P % 2][u], al[u], 0, 0, 0);
             }
-            aload(c + BQ < 8 ? b : b + 1, (c + BQ) % 8);
         }
         const float d4[4] = {f16_bits_to_f32((uint16_t)(r.dw.x & 0xFFFF)), f16_bits_to_f32((uint16_t)(r.dw.x >> 16)),
                              f16_bits_to_f32((uint16_t)(r.dw.y & 0xFFFF)), f16_bits_to_f32((uint16_t)(r.dw.y >> 16))};
@@ -858,10 +927,10 @@ __device__ __forceinline__ void fast_tile_range(const BatchParams &p, int lane, 
             }
     };
     if constexpr (LDSA) {
-        // the class planes come from LDS (lgkmcnt), so the next block's
-        // weights can be in flight a whole block ahead without a class-plane
-        // wait also waiting for them; the scheduling barriers keep the
-        // compiler from sinking those loads back to their first use
+        // the planes come from LDS (lgkmcnt), so the next block's weights can
+        // be in flight a whole block ahead without a plane's wait also waiting
+        // for them; the scheduling barriers keep the compiler from sinking
+        // those loads back to their first use
         W ra, rb;
         wload(ra, b0);
         for (int b = b0; b < b1; b += 2) {
@@ -875,42 +944,9 @@ __device__ __forceinline__ void fast_tile_range(const BatchParams &p, int lane, 
         }
     } else {
         for (int b = b0; b < b1; ++b) {
-            const uint8_t *sg = seg + (size_t)b * SEG_BYTES;
-            const uint4 q0 = *(const uint4 *)(sg + 16 * lane);
-            const uint4 q1 = *(const uint4 *)(sg + SEG_PART + 16 * lane);
-            const uint4 q2 = *(const uint4 *)(sg + 2 * SEG_PART + 16 * lane);
-            const uint32_t scw = *(const uint32_t *)(sg + SEG_SC + 4 * lane);
-            const uint2 dw = *(const uint2 *)(sg + SEG_D + 8 * s);
-            float adb[NC];
-#pragma unroll
-            for (int u = 0; u < NC; ++u) adb[u] = ad[u * chunk_d + (size_t)b * CHUNK_TOKENS];
-            const uint32_t nib[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-            const uint32_t hb[4] = {q2.x, q2.y, q2.z, q2.w};
-            const FoldScales fs = fold_scales(scw);
-            const v4i zero = {0, 0, 0, 0};
-            v4i ah[NC], al[NC];
-#pragma unroll
-            for (int u = 0; u < NC; ++u) ah[u] = al[u] = zero;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                long a_lo, a_hi;
-                fold_digits((uint64_t)unpack_codes(nib, hb, c), fs, a_lo, a_hi);
-#pragma unroll
-                for (int u = 0; u < NC; ++u) {
-                    ah[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, act[c % BQ][u], ah[u], 0, 0, 0);
-                    al[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, act[c % BQ][u], al[u], 0, 0, 0);
-                }
-                aload(c + BQ < 8 ? b : b + 1, (c + BQ) % 8);
-            }
-            const float d4[4] = {f16_bits_to_f32((uint16_t)(dw.x & 0xFFFF)), f16_bits_to_f32((uint16_t)(dw.x >> 16)),
-                                 f16_bits_to_f32((uint16_t)(dw.y & 0xFFFF)), f16_bits_to_f32((uint16_t)(dw.y >> 16))};
-#pragma unroll
-            for (int u = 0; u < NC; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int aux = ah[u][v] * 256 + al[u][v];
-                    acc[u][v] = __builtin_fmaf(d4[v] * adb[u], (float)aux, acc[u][v]);
-                }
+            W r;
+            wload(r, b);
+            compute(r, b);
         }
     }
 }
@@ -961,7 +997,7 @@ __global__ __launch_bounds__(256) void q6k_mv_batched_fast(BatchParams pk) {
     if constexpr (LDSA) {
         const int n16 = p.blocks * CHUNK_BLOCK_BYTES / 16;
         const uint4 *src = (const uint4 *)p.act_q;
-        for (int i = threadIdx.x; i < n16; i += blockDim.x) g_act_lds[i] = src[act_lds_src(i) / 16];
+        for (int i = threadIdx.x; i < n16; i += blockDim.x) g_act_lds[i] = src[i];
         __syncthreads();
         if (live && b0 < b1) fast_tile_range<1, true>(p, lane, t, 0, expert, b0, b1, acc);
     } else if (live && b0 < b1) {
@@ -1033,6 +1069,308 @@ __global__ __launch_bounds__(256) void q6k_mv_batched_fast(BatchParams pk) {
 // computed; one barrier per block hands the buffer over.
 using lds_ptr = __attribute__((address_space(3))) void *;
 
+// One group of tokens against few tiles (Q, K, V or an output projection of a few
+// sequences): a workgroup per (chunk, tile), wave P on classes 2P and 2P + 1
+// alone. Each class's sum stays with one wave, block after block, and one
+// thread per output adds the eight in class order, so the bits are those of
+// q6k_mv_batched; the chip gets four times the waves, each with a quarter
+// of the chain (QKV of 5120 x 2048 on 5 sequences: 16.5 -> 14.4 us a call, norm and
+// quants included).
+__global__ __launch_bounds__(256) void q6k_mv_batched_classes(BatchParams pk) {
+    __shared__ float part[8][4][64];  // [class][v][lane]
+    const int lane = threadIdx.x & 63, P = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    BatchParams p;
+    const int item = batch_item(pk, p, (int)blockIdx.x);
+    const int t = item % p.tiles, chunk = item / p.tiles;
+    if (CHUNK_TOKENS * chunk >= p.single_count) return;
+    const uint8_t *seg = p.w + (size_t)t * p.blocks * SEG_BYTES;
+    const int8_t *aq = p.act_q + (size_t)chunk * p.blocks * CHUNK_BLOCK_BYTES + 1024 * P + 16 * lane;
+    const float *ad = p.act_d + (size_t)chunk * p.blocks * CHUNK_TOKENS + (lane & 15);
+    struct Regs {
+        uint2 nib;
+        uint32_t hb, scw;
+        uint2 dw;
+        v4i a;
+        float ad;
+    };
+    constexpr int B = 4;  // blocks per batch of loads, two batches in turn
+    Regs ra[B], rb[B];
+    const auto load = [&](Regs (&r)[B], int b0) {
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            const int b = min(b0 + k, p.blocks - 1);
+            const uint8_t *sg = seg + (size_t)b * SEG_BYTES;
+            r[k].nib = *(const uint2 *)(sg + (P >> 1) * SEG_PART + 16 * lane + 8 * (P & 1));
+            r[k].hb = *(const uint32_t *)(sg + 2 * SEG_PART + 16 * lane + 4 * P);
+            r[k].scw = *(const uint32_t *)(sg + SEG_SC + 4 * lane);
+            r[k].dw = *(const uint2 *)(sg + SEG_D + 8 * (lane >> 4));
+            r[k].a = *(const v4i *)(aq + (size_t)b * CHUNK_BLOCK_BYTES);
+            r[k].ad = ad[b * CHUNK_TOKENS];
+        }
+    };
+    float sums[2][4] = {};
+    const auto add = [&](const Regs (&r)[B], int b0) {
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            if (b0 + k < p.blocks) {
+                const uint32_t nib[8] = {r[k].nib.x, r[k].nib.y}, hb[4] = {r[k].hb};
+                const FoldScales fs = fold_scales(r[k].scw);
+                const uint16_t dh[4] = {(uint16_t)(r[k].dw.x & 0xFFFF), (uint16_t)(r[k].dw.x >> 16),
+                                        (uint16_t)(r[k].dw.y & 0xFFFF), (uint16_t)(r[k].dw.y >> 16)};
+                const v4i zero = {0, 0, 0, 0};
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    long a_lo, a_hi;
+                    fold_digits((uint64_t)unpack_codes(nib, hb, j), fs, a_lo, a_hi);
+                    const long av = plane_half(r[k].a, j);
+                    const v4i hi = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, av, zero, 0, 0, 0);
+                    const v4i lo = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, av, zero, 0, 0, 0);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int aux = hi[v] * 256 + lo[v];
+                        sums[j][v] = sums[j][v] + f16_bits_to_f32(dh[v]) * r[k].ad * (float)aux;
+                    }
+                }
+            }
+        }
+    };
+    load(ra, 0);
+    for (int b = 0; b < p.blocks; b += 2 * B) {
+        load(rb, b + B);
+        add(ra, b);
+        load(ra, b + 2 * B);
+        add(rb, b + B);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) part[2 * P + j][v][lane] = sums[j][v];
+    __syncthreads();
+    // wave v stores the rows 4s + v
+    const int tok = 16 * chunk + (lane & 15), row = t * TILE_ROWS + 4 * (lane >> 4) + P;
+    if (tok < p.single_count && row < p.rows) {
+        float tot = -0.0f;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) tot = tot + part[c][P][lane];
+        p.y[(size_t)(p.pair_out ? p.pair_out[tok] : tok) * p.ldy + row] = tot;
+    }
+}
+
+// A twin's (or chunk's) planes staged in LDS for 4 tiles, as in
+// q6k_mv_batched_fast_staged below: a plane is read from L2 once per 4 tiles
+// instead of once per tile, and the loop keeps no planes in flight in registers
+// (512 tokens, skewed routing: 282 -> 262 us a call; 2000: 775 -> 727; still
+// bound by vector issue, the fold per twin and the ordered sums per chunk).
+template <int NC, bool PF = false>
+__device__ __forceinline__ void exact_tile_staged(const BatchParams &p, const GroupItem &it, int lane, int wave,
+                                                  int t) {
+    const size_t chunk_q = (size_t)p.blocks * CHUNK_BLOCK_BYTES, chunk_d = (size_t)p.blocks * CHUNK_TOKENS;
+    const uint8_t *seg = p.w + (size_t)it.expert * p.expert_stride + (size_t)t * p.blocks * SEG_BYTES;
+    const int8_t *gq = p.act_q + (size_t)it.sub * chunk_q + 1024 * wave + 16 * lane;
+    const float *ad = p.act_d + (size_t)it.sub * chunk_d + (lane & 15);
+    int8_t *lds = (int8_t *)g_act_lds;  // [2][NC][4096]
+    auto stage = [&](int b) {           // plane `wave` of each chunk
+#pragma unroll
+        for (int u = 0; u < NC; ++u)
+            __builtin_amdgcn_global_load_lds((const void *)(gq + u * chunk_q + (size_t)b * CHUNK_BLOCK_BYTES),
+                                             (lds_ptr)(lds + ((b & 1) * NC + u) * CHUNK_BLOCK_BYTES + 1024 * wave),
+                                             16, 0, 0);
+    };
+    float sums[NC][8][4];
+#pragma unroll
+    for (int u = 0; u < NC; ++u)
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sums[u][c][v] = 0.0f;
+    struct R {
+        TileRegs t;
+        float adb[NC];
+    } ra, rb;
+    const int last = p.blocks - 1;
+    const auto load = [&](R &r, int b) {
+        tile_load(r.t, seg + (size_t)b * SEG_BYTES, lane);
+#pragma unroll
+        for (int u = 0; u < NC; ++u) r.adb[u] = ad[u * chunk_d + (size_t)b * CHUNK_TOKENS];
+    };
+    // block b's planes (and weights) have landed, and the other buffer is read
+    const auto handover = [&]() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+    stage(0);
+    if constexpr (PF) {
+        load(ra, 0);
+        // the next block's weights in flight too, where registers allow
+        for (int b = 0; b < p.blocks; b += 2) {
+            handover();
+            if (b < last) stage(b + 1);
+            load(rb, min(b + 1, last));
+            __builtin_amdgcn_sched_barrier(0);
+            tile_block<NC>(ra.t, ra.adb, lds + 16 * lane, sums);
+            if (b == last) break;
+            handover();
+            if (b + 1 < last) stage(b + 2);
+            load(ra, min(b + 2, last));
+            __builtin_amdgcn_sched_barrier(0);
+            tile_block<NC>(rb.t, rb.adb, lds + NC * CHUNK_BLOCK_BYTES + 16 * lane, sums);
+        }
+    } else {
+        for (int b = 0; b < p.blocks; ++b) {
+            load(ra, b);
+            handover();
+            if (b < last) stage(b + 1);
+            tile_block<NC>(ra.t, ra.adb, lds + (b & 1) * NC * CHUNK_BLOCK_BYTES + 16 * lane, sums);
+        }
+    }
+    batched_store<NC>(p, sums, lane, t, it.st, it.count, it.start);
+}
+
+// A group of T <= 2 tokens against a tile, as q6k_mv_b1 does it: the masked
+// activations and the scales after the MFMA, so nothing is folded into the
+// weights and no token slot is idle (about 110 and 170 vector instructions per
+// block for 1 and 2 tokens, 330 for a 16-token chunk). The A operand of class c
+// is this lane's 8 bytes of the chunk's plane, kept where they belong to scale
+// group n.
+template <int T>
+__device__ __forceinline__ void few_tile(const BatchParams &p, const GroupItem &it, int lane, int t) {
+    const int n = lane & 15, s = lane >> 4;
+    const uint8_t *seg = p.w + (size_t)it.expert * p.expert_stride + (size_t)t * p.blocks * SEG_BYTES;
+    const int8_t *aq = p.act_q + (size_t)it.sub * p.blocks * CHUNK_BLOCK_BYTES + 256 * s;
+    const float *ad = p.act_d + (size_t)it.sub * p.blocks * CHUNK_TOKENS;
+    const uint64_t mask = (n >> 2) == s ? 0xFFFFull << (16 * (n & 3)) : 0ull;
+    struct Regs {
+        uint4 q0, q1, q2;
+        uint32_t scw;
+        uint16_t dh;
+        v4i a[T][4];
+        float ad[T];
+    } ra, rb;
+    const auto load = [&](Regs &r, int b) {
+        const uint8_t *sg = seg + (size_t)b * SEG_BYTES;
+        r.q0 = *(const uint4 *)(sg + 16 * lane);
+        r.q1 = *(const uint4 *)(sg + SEG_PART + 16 * lane);
+        r.q2 = *(const uint4 *)(sg + 2 * SEG_PART + 16 * lane);
+        r.scw = *(const uint32_t *)(sg + SEG_SC + 4 * lane);
+        r.dh = *(const uint16_t *)(sg + SEG_D + 2 * n);
+#pragma unroll
+        for (int k = 0; k < T; ++k) {
+#pragma unroll
+            for (int P = 0; P < 4; ++P)
+                r.a[k][P] = *(const v4i *)(aq + (size_t)b * CHUNK_BLOCK_BYTES + 1024 * P + 16 * k);
+            r.ad[k] = ad[b * CHUNK_TOKENS + k];
+        }
+    };
+    float se[T], so[T];  // classes 2s and 2s+1 of row n
+#pragma unroll
+    for (int k = 0; k < T; ++k) se[k] = so[k] = 0.0f;
+    const auto add = [&](const Regs &r) {
+        const uint32_t nib[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
+        const uint32_t hb[4] = {r.q2.x, r.q2.y, r.q2.z, r.q2.w};
+        const v4i zero = {0, 0, 0, 0};
+        const int sc0 = __builtin_amdgcn_sbfe(r.scw, 0, 8), sc1 = __builtin_amdgcn_sbfe(r.scw, 8, 8);
+        const int sc2 = __builtin_amdgcn_sbfe(r.scw, 16, 8), sc3 = __builtin_amdgcn_sbfe(r.scw, 24, 8);
+        int acc[T][8];
+        v4i d[2][T];
+        const auto dots = [&](int c) {
+            const long codes = unpack_codes(nib, hb, c);
+#pragma unroll
+            for (int k = 0; k < T; ++k) {
+                const long am = plane_half(r.a[k][c >> 1], c & 1) & (long)mask;
+                const v4i kc = __builtin_amdgcn_mfma_i32_16x16x32_i8(am, NEG32_BYTES, zero, 0, 0, 0);
+                d[c & 1][k] = __builtin_amdgcn_mfma_i32_16x16x32_i8(am, codes, kc, 0, 0, 0);
+            }
+        };
+        dots(0);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            if (c + 1 < 8) dots(c + 1);
+#pragma unroll
+            for (int k = 0; k < T; ++k) {
+                int v = __mul24(sc0, d[c & 1][k][0]);
+                v = __mul24(sc1, d[c & 1][k][1]) + v;
+                v = __mul24(sc2, d[c & 1][k][2]) + v;
+                acc[k][c] = __mul24(sc3, d[c & 1][k][3]) + v;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < T; ++k) {
+            int ae, ao;
+            reduce_classes(acc[k], ae, ao);
+            const float dd = f16_bits_to_f32(r.dh) * r.ad[k];
+            se[k] = se[k] + dd * (float)ae;
+            so[k] = so[k] + dd * (float)ao;
+        }
+    };
+    const int last = p.blocks - 1;
+    load(ra, 0);
+    for (int b = 0; b < p.blocks; b += 2) {
+        load(rb, min(b + 1, last));
+        add(ra);
+        if (b == last) break;
+        load(ra, min(b + 2, last));
+        add(rb);
+    }
+    const int row = t * TILE_ROWS + n;
+#pragma unroll
+    for (int k = 0; k < T; ++k) {
+        // lane (n, 0) adds the eight class sums in class order (dot.rs:195)
+        float tot = -0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            tot = tot + __shfl(se[k], n + 16 * q, WAVE);
+            tot = tot + __shfl(so[k], n + 16 * q, WAVE);
+        }
+        if (s == 0 && row < p.rows)
+            p.y[(size_t)(p.pair_out ? p.pair_out[it.start + k] : it.start + k) * p.ldy + row] = tot;
+    }
+}
+
+// (tiles % 4 == 0: the workgroup's 4 items share their twin, so its exits are
+// uniform and no barrier is skipped by some waves only)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void q6k_mv_batched_twin_staged(BatchParams pk) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    BatchParams p;
+    const int item = batch_item(pk, p);
+    if (item >= p.items_per_mat) return;
+    const GroupItem it = p.twin_info[item / p.tiles];
+    if (it.expert < 0) return;
+    if (it.twin2) exact_tile_staged<2>(p, it, lane, wave, item % p.tiles);
+    else exact_tile_staged<1>(p, it, lane, wave, item % p.tiles);
+}
+
+// The same by chunks on one group of tokens (LM head of 151936 rows, 16
+// sequences: 75.7 -> 70.3 us a call; of 32003: 22.4 -> 20.9; QKV of 96 tokens
+// 22.4 -> 21.0, of 512 61.7, 61.8; the whole chunk in LDS before the first
+// block: 73.9, 23.2).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void q6k_mv_batched_staged(BatchParams pk) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    BatchParams p;
+    const int item = batch_item(pk, p);
+    // the grid's rounding to whole workgroups: those waves only stage
+    const bool live = item < p.items_per_mat;
+    const int chunk = live ? item / p.tiles : 0;
+    if (CHUNK_TOKENS * chunk >= p.single_count) return;
+    const GroupItem it = {0, chunk, chunk, live ? p.single_count : 0, 0, 0, 0, 0};
+    exact_tile_staged<1, true>(p, it, lane, wave, live ? item % p.tiles : 0);
+}
+
+// The same by chunks, for calls that leave most experts a token or two.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void q6k_mv_batched_few(BatchParams pk) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    BatchParams p;
+    const int item = batch_item(pk, p);
+    if (item >= p.items_per_mat) return;
+    const GroupItem it = p.sub_info[item / p.tiles];
+    if (it.expert < 0) return;
+    if (it.count == 1) few_tile<1>(p, it, lane, item % p.tiles);
+    else if (it.count == 2) few_tile<2>(p, it, lane, item % p.tiles);
+    else exact_tile_staged<1, true>(p, it, lane, wave, item % p.tiles);
+}
+
 template <int NC>
 __device__ __forceinline__ void fast_tile_staged(const BatchParams &p, int lane, int wave, int t,
                                                  int sub0, int expert, float acc[2][4]) {
@@ -1050,7 +1388,7 @@ __device__ __forceinline__ void fast_tile_staged(const BatchParams &p, int lane,
             const int off = (wave * NC + i) * 1024;  // within the NC x 4 KiB
             const int u = off / CHUNK_BLOCK_BYTES, o = off % CHUNK_BLOCK_BYTES;
             __builtin_amdgcn_global_load_lds(
-                (const void *)(gq + u * chunk_q + (size_t)b * CHUNK_BLOCK_BYTES + act_lds_src(o / 16 + lane)),
+                (const void *)(gq + u * chunk_q + (size_t)b * CHUNK_BLOCK_BYTES + o + 16 * lane),
                 (lds_ptr)(lds + (b & 1) * BUF + off), 16, 0, 0);
         }
     };
@@ -1071,7 +1409,7 @@ __device__ __forceinline__ void fast_tile_staged(const BatchParams &p, int lane,
         for (int u = 0; u < NC; ++u) r.adb[u] = ad[u * chunk_d + (size_t)b * CHUNK_TOKENS];
     };
     auto compute = [&](const W &r, int b) {
-        const int8_t *aq = lds + (b & 1) * BUF + act_lds_byte(n, s);
+        const int8_t *aq = lds + (b & 1) * BUF + 16 * lane;
         const uint32_t nib[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
         const uint32_t hb[4] = {r.q2.x, r.q2.y, r.q2.z, r.q2.w};
         const FoldScales fs = fold_scales(r.scw);
@@ -1080,14 +1418,14 @@ __device__ __forceinline__ void fast_tile_staged(const BatchParams &p, int lane,
 #pragma unroll
         for (int u = 0; u < NC; ++u) ah[u] = al[u] = zero;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            long a_lo, a_hi;
-            fold_digits((uint64_t)unpack_codes(nib, hb, c), fs, a_lo, a_hi);
+        for (int P = 0; P < 4; ++P) {
+            v4i a_lo, a_hi;
+            fold_pair(nib, hb, P, fs, a_lo, a_hi);
 #pragma unroll
             for (int u = 0; u < NC; ++u) {
-                const long av = *(const long *)(aq + u * CHUNK_BLOCK_BYTES + 512 * c);
-                ah[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, av, ah[u], 0, 0, 0);
-                al[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, av, al[u], 0, 0, 0);
+                const v4i av = *(const v4i *)(aq + u * CHUNK_BLOCK_BYTES + 1024 * P);
+                ah[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_hi, av, ah[u], 0, 0, 0);
+                al[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_lo, av, al[u], 0, 0, 0);
             }
         }
         const float d4[4] = {f16_bits_to_f32((uint16_t)(r.dw.x & 0xFFFF)), f16_bits_to_f32((uint16_t)(r.dw.x >> 16)),
@@ -1632,12 +1970,30 @@ int launch_q6k_mv_routed(const void *w, const void *w_b, size_t expert_stride,
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+namespace {
+// The exact kernels on one group of tokens, items = tiles x chunks in all.
+int launch_one_group(const BatchParams &p, long items, hipStream_t st) {
+    const dim3 grid((unsigned)((items + 3) / 4));
+    // the 4 tiles of a workgroup share a chunk
+    bool even = p.tiles % 4 == 0;
+    for (int i = 1; i < p.n_segs; ++i) even = even && p.segs[i].tiles % 4 == 0;
+    // half a wave per SIMD or less (us per call with the norm and the quants, a
+    // wave per item -> four: 320 items 15.9 -> 14.4, 640 16.3 -> 16.8)
+    if (items <= 512 && !p.amax_v)
+        hipLaunchKernelGGL(q6k_mv_batched_classes, dim3((unsigned)items), dim3(256), 0, st, p);
+    else if (p.single_count <= CHUNK_TOKENS || even)
+        hipLaunchKernelGGL(q6k_mv_batched_staged, grid, dim3(256), 2 * CHUNK_BLOCK_BYTES, st, p);
+    else hipLaunchKernelGGL(q6k_mv_batched, grid, dim3(256), 0, st, p);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+}  // namespace
+
 int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *grp_expert,
                           const int32_t *grp_start, const int32_t *grp_count,
                           const int32_t *sub_start, const int32_t *pair_out, const int8_t *act_q,
                           const float *act_d, float *y, int ldy, int rows, int blocks,
                           int n_groups, int max_chunks, hipStream_t st, float *amax_v,
-                          int *amax_i, bool group_tables, const void *w2, float *y2, bool fast) {
+                          int *amax_i, bool group_tables, const void *w2, float *y2, bool fast, bool few) {
     if (amax_v && grp_expert) return -1;
     // every item of the grids below indexes a record below max_chunks when
     // max_chunks >= n_groups (twins: ceil((max_chunks + n_groups) / 2) items)
@@ -1696,19 +2052,29 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
         else hipLaunchKernelGGL((q6k_mv_batched_fast<1, false>), dim3(grid), dim3(256), 0, st, p);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
+    if (group_tables && few && g_tune_batched_twin && (rows + TILE_ROWS - 1) / TILE_ROWS % 4 == 0) {
+        const long items = (long)p.tiles * max_chunks;
+        p.items_per_mat = (int)items;
+        hipLaunchKernelGGL(q6k_mv_batched_few, dim3((unsigned)((w2 ? 2 * items : items) / 4)), dim3(256),
+                           2 * CHUNK_BLOCK_BYTES, st, p);
+        return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
     if (grp_expert && g_tune_batched_twin) {
         // twins: sum of ceil(ch/2) <= (sum of ch + n_groups) / 2
         const long items = (long)p.tiles * ((max_chunks + n_groups + 1) / 2);
         if (items <= 0) return 0;
         p.items_per_mat = (int)items;
         const long all = w2 ? 2 * items : items;
-        hipLaunchKernelGGL(q6k_mv_batched_twin, dim3((unsigned)((all + 3) / 4)), dim3(256), 0, st, p);
+        if (group_tables && p.tiles % 4 == 0)
+            hipLaunchKernelGGL(q6k_mv_batched_twin_staged, dim3((unsigned)(all / 4)), dim3(256), 4 * CHUNK_BLOCK_BYTES, st, p);
+        else hipLaunchKernelGGL(q6k_mv_batched_twin, dim3((unsigned)((all + 3) / 4)), dim3(256), 0, st, p);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
     const long items = (long)p.tiles * max_chunks;
     if (items <= 0) return 0;
     p.items_per_mat = (int)items;
     const long all = w2 ? 2 * items : items;
+    if (!grp_expert) return launch_one_group(p, all, st);
     hipLaunchKernelGGL(q6k_mv_batched, dim3((unsigned)((all + 3) / 4)), dim3(256), 0, st, p);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -1740,8 +2106,7 @@ int launch_q6k_mv_batched_x3(const void *const w[3], float *const y[3], const in
     p.act_d = act_d;
     p.blocks = blocks;
     p.single_count = nseq;  // one group (expert 0) of nseq tokens
-    hipLaunchKernelGGL(q6k_mv_batched, dim3((unsigned)((first + 3) / 4)), dim3(256), 0, st, p);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    return launch_one_group(p, first, st);
 }
 
 int launch_q6k_down_combine(const void *w, size_t expert_stride, const int32_t *ids,

@@ -7,6 +7,7 @@
 
 #include "common.hpp"
 #include "expf_ref.h"
+#include "launch.hpp"
 
 namespace llamd {
 
@@ -64,16 +65,19 @@ __device__ __forceinline__ void quantize_wave(const float v[4], int lane, int8_t
 
 // ---- token-chunked activations (the batched matvec's operand layout) -----
 // 16 token slots form a chunk; block b of chunk k occupies 4 KiB at
-// (k * blocks + b) * 4096, holding class plane c (weights e with e % 8 == c)
-// at c * 512, token n of the chunk at n * 32 within it, and weight 8 m + c
-// at byte m. One MFMA operand load of a class is then one contiguous 512-B
-// read for the whole wave. The scales sit at d[(k * blocks + b) * 16 + n].
+// (k * blocks + b) * 4096, holding four planes of two classes (weights e with
+// e % 8 == 2 P or 2 P + 1) at P * 1024. A plane is 64 units of 16 bytes, unit
+// n + 16 s for token n and quarter s: weights 8 m + 2 P for m = 8 s .. 8 s + 7,
+// then 8 m + 2 P + 1 for the same m. That is the MFMA operand of lane n + 16 s,
+// so a wave reads a plane as one contiguous KiB (one 16-byte load a lane, from
+// LDS without bank conflicts), whole for the 64-deep MFMA of two classes or a
+// half per class. The scales sit at d[(k * blocks + b) * 16 + n].
 constexpr int CHUNK_TOKENS = 16;
 constexpr int CHUNK_BLOCK_BYTES = 8 * 512;
 
 // The wave's quants regrouped for the chunked layout: lane L ends up with
-// the 4 bytes of class plane L / 8 at bytes 4 (L % 8) .. +3 of the token's
-// 32 -- elements 8k + L / 8 for k = 4 (L % 8) .. +3 -- gathered from the
+// 4 bytes of class L / 8 of the token -- elements 8k + L / 8 for k = 4 (L % 8)
+// .. +3, which lie together at chunk_byte of the first -- gathered from the
 // lanes that hold them (lane e / 4 holds element e), so each lane then
 // stores one dword per destination instead of four scattered bytes.
 __device__ __forceinline__ uint32_t chunk_dword(const int q[4], int lane) {
@@ -93,8 +97,8 @@ __device__ __forceinline__ void store_chunk(uint32_t dword, float dv, int lane, 
                                             float *cd, int slot, int b, int blocks) {
     if (slot < 0) return;  // a pair with no expert (out-of-range id)
     const size_t base = ((size_t)(slot / CHUNK_TOKENS) * blocks + b);
-    int8_t *dst = cq + base * CHUNK_BLOCK_BYTES + (slot % CHUNK_TOKENS) * 32;
-    *(uint32_t *)(dst + (lane >> 3) * 512 + 4 * (lane & 7)) = dword;
+    int8_t *dst = cq + base * CHUNK_BLOCK_BYTES;
+    *(uint32_t *)(dst + chunk_byte(32 * (lane & 7) + (lane >> 3), slot % CHUNK_TOKENS)) = dword;
     if (lane == 0) cd[base * CHUNK_TOKENS + slot % CHUNK_TOKENS] = dv;
 }
 
