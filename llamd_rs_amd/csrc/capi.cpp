@@ -1059,6 +1059,14 @@ int llamd_hip_moe_stats(void *h, int *calls, int *exact_calls) {
 
 namespace {
 
+// The REDUCTION GEMMs on wide units (launch_q6k_mv_batched_wide) from 8 pairs
+// per expert on. Measured per call (us, twins staged in LDS -> wide units; 128
+// experts, top 8): 24 tokens 105 -> 106, 45 101 -> 101, 100 124 -> 124, 200
+// 141 -> 132, 512 201..205 -> 161..182, 1000 309 -> 249, 2000 538 -> 367.
+bool moe_wide(const MoeLayer *m, int n_pairs) {
+    return n_pairs / 8 >= m->n_expert && q6k_wide_fits(m->n_ff, m->be) && q6k_wide_fits(m->n_embd, m->bf);
+}
+
 // The expert-grouped FFN of n_tok tokens with routing ids / weights
 // [n_tok][n_used] on the device; out = res + moe_ffn (res optional).
 int moe_grouped(MoeLayer *m, const float *d_x, const int32_t *d_ids, const float *d_w,
@@ -1073,7 +1081,7 @@ int moe_grouped(MoeLayer *m, const float *d_x, const int32_t *d_ids, const float
         bool ok = m->p_xq.alloc((size_t)chunks * m->be * CHUNK_BLOCK) &&
                   m->p_xd.alloc((size_t)chunks * m->be * CHUNK * 4) &&
                   m->p_grp_e.alloc(m->n_expert * 4) && m->p_grp_s.alloc(m->n_expert * 4) &&
-                  m->p_grp_c.alloc(m->n_expert * 4) && m->p_sub.alloc((group_items_offset(m->n_expert) + 2 * (size_t)chunks * 8) * 4) &&
+                  m->p_grp_c.alloc(m->n_expert * 4) && m->p_sub.alloc(group_table_size(m->n_expert, chunks) * 4) &&
                   m->p_slot.alloc(NP * 4) && m->p_idx.alloc(NP * 4) &&
                   m->p_g.alloc(NP * m->n_ff * 4) && m->p_u.alloc(NP * m->n_ff * 4) &&
                   m->p_aq.alloc((size_t)chunks * m->bf * CHUNK_BLOCK) &&
@@ -1099,6 +1107,20 @@ int moe_grouped(MoeLayer *m, const float *d_x, const int32_t *d_ids, const float
     // Q8_K of every token, written to the chunk slot of each of its n_used pairs
     rc |= launch_q8k_quantize_chunks(d_x, n_tok, m->be, m->p_slot.as<int32_t>(), m->n_used,
                                      m->p_xq.as<int8_t>(), m->p_xd.as<float>(), st);
+    if (fast && moe_wide(m, np)) {
+        // gate, up and SwiGLU in one launch, Q8_K of its rows, down
+        rc |= launch_q6k_mv_batched_wide(m->gate, m->upw, m->sgu, m->p_sub.as<int32_t>(),
+                                         m->p_idx.as<int32_t>(), m->p_xq.as<int8_t>(), m->p_xd.as<float>(),
+                                         m->p_g.as<float>(), m->n_ff, m->be, m->n_expert, max_chunks, st);
+        rc |= launch_q8k_quantize_chunks(m->p_g.as<float>(), np, m->bf, m->p_slot.as<int32_t>(), 1,
+                                         m->p_aq.as<int8_t>(), m->p_ad.as<float>(), st);
+        rc |= launch_q6k_mv_batched_wide(m->downw, nullptr, m->sd, m->p_sub.as<int32_t>(),
+                                         m->p_idx.as<int32_t>(), m->p_aq.as<int8_t>(), m->p_ad.as<float>(),
+                                         m->p_dn.as<float>(), m->n_embd, m->bf, m->n_expert, max_chunks, st);
+        rc |= launch_moe_combine(m->p_dn.as<float>(), d_w, d_res, d_out, m->n_used, m->n_embd, n_tok, st,
+                                 m->p_slot.as<int32_t>());
+        return rc ? fail("moe_prefill: launch failed") : 0;
+    }
     // gate / up: output row = the pair index
     // gate and up in one launch (same shapes, same activations)
     rc |= launch_q6k_mv_batched(m->gate, m->sgu, m->p_grp_e.as<int32_t>(), m->p_grp_s.as<int32_t>(),

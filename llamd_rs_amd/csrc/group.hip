@@ -19,8 +19,9 @@
 //   (chunk sub_start[e] + j / 16, token j % 16 for the j-th pair of expert
 //   e), pair_idx[i] = the pair index t * n_used + k at sorted position i.
 // With max_chunks > 0, sub_start continues with a record per chunk,
-// sub_info[max_chunks], then one per twin, twin_info[max_chunks] (GroupItem,
-// launch.hpp): a wave of the batched kernels reads its work item in one load
+// sub_info[max_chunks], then one per twin, twin_info[max_chunks], then one per
+// wide unit (up to GROUP_WIDE_CHUNKS chunks, an expert's chunks split evenly)
+// (GroupItem, launch.hpp): a wave of the batched kernels reads its work item in one load
 // instead of a binary search of dependent loads and the group's fields.
 #include "common.hpp"
 #include "launch.hpp"
@@ -34,25 +35,29 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
                                                   int n_expert, int32_t *grp_expert,
                                                   int32_t *grp_start, int32_t *grp_count,
                                                   int32_t *sub_start, int32_t *slot_of_pair,
-                                                  int32_t *pair_idx, int max_chunks) {
+                                                  int32_t *pair_idx, int max_chunks, int max_sorted) {
     __shared__ int sub_lds[GROUP_MAX_EXPERTS];
     __shared__ int start_lds[GROUP_MAX_EXPERTS];
     (void)n_used;
     __shared__ int hist[GROUP_MAX_EXPERTS];
     __shared__ int cursor[GROUP_MAX_EXPERTS];
-    __shared__ int totals[2];  // chunks, twins
+    constexpr int PB = 8;
+    const bool once = n_pairs <= PB * (int)blockDim.x;
+    // the sorted pairs of a long prompt: scattered here, then written in order
+    // (2000 tokens of 8: 18 -> 15 us; nothing to gain up to 8192 pairs)
+    extern __shared__ int32_t sorted_lds[];
+    int32_t *sorted = once || n_pairs > max_sorted ? nullptr : sorted_lds;
+    __shared__ int totals[4];  // chunks, twins, pairs in a group, wide units
     const int tid = threadIdx.x;
     for (int e = tid; e < n_expert; e += blockDim.x) hist[e] = 0;
     __syncthreads();
     // a pair whose id is outside [0, n_expert) joins no group: its slot is -1,
     // which the chunk quantizers skip and the combine counts as no term
     // ids in batches of PB per thread, all of a batch's loads in flight
-    // before its first atomic (one memory round trip per batch, not per id)
-    constexpr int PB = 8;
-    // the last batch's ids stay in registers for the scatter below (with up
-    // to PB * blockDim.x pairs, the only batch: no second round trip)
-    int eid[PB];
-    int last_base = 0;
+    // before its first atomic (one memory round trip per batch, not per id).
+    // An id's place within its expert is what its count's increment returns;
+    // it stays in a register, with the id, for the scatter below.
+    int eid[PB], rank[PB];
     for (int base = 0; base < n_pairs; base += PB * (int)blockDim.x) {
 #pragma unroll
         for (int k = 0; k < PB; ++k) {
@@ -61,28 +66,31 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
         }
 #pragma unroll
         for (int k = 0; k < PB; ++k)
-            if ((unsigned)eid[k] < (unsigned)n_expert) atomicAdd(&hist[eid[k]], 1);
-        last_base = base;
+            if ((unsigned)eid[k] < (unsigned)n_expert) rank[k] = atomicAdd(&hist[eid[k]], 1);
     }
     __syncthreads();
     // exclusive prefix sums over experts (thread e owns expert e) of the
     // pair counts and of the 16-token chunk counts
     __shared__ int wsum_c[GROUP_MAX_EXPERTS / WAVE], wsum_s[GROUP_MAX_EXPERTS / WAVE],
-        wsum_t[GROUP_MAX_EXPERTS / WAVE];
+        wsum_t[GROUP_MAX_EXPERTS / WAVE], wsum_u[GROUP_MAX_EXPERTS / WAVE];
     const int lane = tid & 63, wave = tid >> 6;
     const int c = tid < n_expert ? hist[tid] : 0, ch = (c + 15) / 16, tw = (ch + 1) / 2;
+    const int wu = (ch + GROUP_WIDE_CHUNKS - 1) / GROUP_WIDE_CHUNKS;
     const int ic = wave_incl_sum_i(c), is = wave_incl_sum_i(ch), it = wave_incl_sum_i(tw);
+    const int iu = wave_incl_sum_i(wu);
     if (lane == WAVE - 1) {
         wsum_c[wave] = ic;
         wsum_s[wave] = is;
         wsum_t[wave] = it;
+        wsum_u[wave] = iu;
     }
     __syncthreads();
-    int start = ic - c, sub = is - ch, tst = it - tw;
+    int start = ic - c, sub = is - ch, tst = it - tw, ust = iu - wu;
     for (int w = 0; w < wave; ++w) {
         start += wsum_c[w];
         sub += wsum_s[w];
         tst += wsum_t[w];
+        ust += wsum_u[w];
     }
     if (tid < n_expert) {
         grp_expert[tid] = tid;
@@ -92,12 +100,14 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
         sub_start[n_expert + 1 + tid] = tst;
         sub_lds[tid] = sub;
         start_lds[tid] = start;
-        cursor[tid] = start;
+        cursor[tid] = 0;
         if (tid == n_expert - 1) {
             sub_start[n_expert] = sub + ch;
             sub_start[2 * n_expert + 1] = tst + tw;
             totals[0] = sub + ch;
             totals[1] = tst + tw;
+            totals[2] = start + c;
+            totals[3] = ust + wu;
         }
         if (max_chunks > 0) {
             GroupItem *sub_info = (GroupItem *)(sub_start + group_items_offset(n_expert));
@@ -106,6 +116,12 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
                 sub_info[sub + j] = GroupItem{tid, j, sub + j, c, start, 0, 0, 0};
             for (int j = 0; j < tw; ++j)
                 twin_info[tst + j] = GroupItem{tid, 2 * j, sub + 2 * j, c, start, 2 * j + 1 < ch, 0, 0};
+            GroupItem *wide_info = twin_info + max_chunks;
+            for (int j = 0, at = 0; j < wu; ++j) {
+                const int nc = ch / wu + (j < ch % wu);
+                wide_info[ust + j] = GroupItem{tid, at, sub + at, c, start, nc, 0, 0};
+                at += nc;
+            }
         }
     }
     __syncthreads();
@@ -118,15 +134,21 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
             sub_info[i] = GroupItem{-1, 0, 0, 0, 0, 0, 0, 0};
         for (int i = totals[1] + tid; i < max_chunks; i += blockDim.x)
             twin_info[i] = GroupItem{-1, 0, 0, 0, 0, 0, 0, 0};
+        GroupItem *wide_info = twin_info + max_chunks;
+        for (int i = totals[3] + tid; i < group_wide_units(n_expert, max_chunks); i += blockDim.x)
+            wide_info[i] = GroupItem{-1, 0, 0, 0, 0, 0, 0, 0};
     }
-    // batches in reverse, the one still in registers first
-    for (int base = last_base; base >= 0 && n_pairs > 0; base -= PB * (int)blockDim.x) {
-        if (base != last_base) {
+    for (int base = 0; base < n_pairs; base += PB * (int)blockDim.x) {
+        if (!once) {
+            // more pairs than registers: the ids and their places again
 #pragma unroll
             for (int k = 0; k < PB; ++k) {
                 const int p = base + k * (int)blockDim.x + tid;
                 eid[k] = p < n_pairs ? ids[p] : -1;
             }
+#pragma unroll
+            for (int k = 0; k < PB; ++k)
+                if ((unsigned)eid[k] < (unsigned)n_expert) rank[k] = atomicAdd(&cursor[eid[k]], 1);
         }
 #pragma unroll
         for (int k = 0; k < PB; ++k) {
@@ -137,11 +159,14 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
                 slot_of_pair[p] = -1;
                 continue;
             }
-            const int pos = atomicAdd(&cursor[e], 1);
-            const int j = pos - start_lds[e];
+            const int j = rank[k];
             slot_of_pair[p] = (sub_lds[e] + j / 16) * 16 + j % 16;
-            pair_idx[pos] = p;
+            (sorted ? sorted : pair_idx)[start_lds[e] + j] = p;
         }
+    }
+    if (sorted) {
+        __syncthreads();
+        for (int i = tid; i < totals[2]; i += blockDim.x) pair_idx[i] = sorted[i];
     }
 }
 
@@ -152,9 +177,14 @@ int launch_moe_group(const int32_t *ids, int n_pairs, int n_used, int n_expert,
                      int32_t *sub_start, int32_t *slot_of_pair, int32_t *pair_idx,
                      hipStream_t st, int max_chunks) {
     if (n_expert > GROUP_MAX_EXPERTS || n_expert <= 0 || max_chunks < 0) return -1;
-    hipLaunchKernelGGL(moe_group, dim3(1), dim3(1024), 0, st, ids, n_pairs, n_used, n_expert,
+    const int max_sorted = 24576;
+    const size_t lds = n_pairs > 8192 && n_pairs <= max_sorted ? (size_t)n_pairs * 4 : 0;
+    static const hipError_t ok = hipFuncSetAttribute((const void *)moe_group, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     max_sorted * 4);
+    if (ok != hipSuccess) return -1;
+    hipLaunchKernelGGL(moe_group, dim3(1), dim3(1024), lds, st, ids, n_pairs, n_used, n_expert,
                        grp_expert, grp_start, grp_count, sub_start, slot_of_pair, pair_idx,
-                       max_chunks);
+                       max_chunks, max_sorted);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -124,6 +124,16 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
 // class sums; outputs within REDUCTION of dot_q6k_q8k, not bit-identical).
 // few: exact grouped calls (with group_tables) that leave most groups a token
 // or two.
+
+// The REDUCTION GEMM of launch_q6k_mv_batched for many tokens per expert, on
+// moe_group's units of up to GROUP_WIDE_CHUNKS chunks (same sums, same bits).
+// w2 set: y = silu(w . a) * (w2 . a) instead. y [pairs][rows], 16-byte aligned.
+constexpr int WIDE_MAX_BLOCKS = 16;
+bool q6k_wide_fits(int rows, int blocks);
+int launch_q6k_mv_batched_wide(const void *w, const void *w2, size_t expert_stride,
+                               const int32_t *sub_start, const int32_t *pair_out,
+                               const int8_t *act_q, const float *act_d, float *y, int rows,
+                               int blocks, int n_groups, int max_chunks, hipStream_t st);
 // Up to three matrices with their own row counts (Q, K, V) against the same
 // nseq token-chunked activations, one launch: y[i] [nseq][rows[i]].
 int launch_q6k_mv_batched_x3(const void *const w[3], float *const y[3], const int rows[3], int n_mat,
@@ -165,8 +175,8 @@ int launch_swiglu_q8k_chunks(const float *gate, const float *up, int rows, int b
 // moe grouping (group.hip): counting sort of the (token, k) pairs by expert.
 // Outputs grp_* per expert, sub_start (prefix of ceil(count/16), then the
 // twin prefix of ceil(chunks/2): 2 * (n_expert + 1) entries; with
-// max_chunks > 0 then a GroupItem per chunk and per twin, from
-// group_items_offset(n_expert), 2 * max_chunks records), for each
+// max_chunks > 0 then a GroupItem per chunk, per twin and per wide unit, from
+// group_items_offset(n_expert): group_table_size entries in all), for each
 // pair p = token * n_used + k its chunk slot slot_of_pair[p], and for each
 // sorted position its pair index pair_idx.
 // One work item of the expert-grouped batched kernels: a 16-token chunk, or a
@@ -177,12 +187,23 @@ struct __attribute__((aligned(32))) GroupItem {
     int32_t sub;     // first chunk's global index (its activation chunk)
     int32_t count;   // pairs in the group
     int32_t start;   // the group's first sorted pair
-    int32_t twin2;   // twins: 1 when the second chunk exists
+    int32_t twin2;   // twins: 1 when the second chunk exists; wide units: chunks
     int32_t pad0, pad1;
 };
 // The records start at this int32 offset of sub_start (32-byte aligned
 // when sub_start is).
 constexpr size_t group_items_offset(int n_expert) { return ((2 * (size_t)(n_expert + 1)) + 7) & ~(size_t)7; }
+// Wide units: up to this many consecutive chunks of one expert, and the
+// records (a multiple of 8) that any grouping into max_chunks chunks takes.
+constexpr int GROUP_WIDE_CHUNKS = 8;
+constexpr int group_wide_units(int n_expert, int max_chunks) {
+    return (max_chunks / GROUP_WIDE_CHUNKS + n_expert + 7) / 8 * 8;
+}
+// int32 entries of sub_start with its records
+constexpr size_t group_table_size(int n_expert, int max_chunks) {
+    return group_items_offset(n_expert) +
+           (2 * (size_t)max_chunks + group_wide_units(n_expert, max_chunks)) * sizeof(GroupItem) / 4;
+}
 int launch_moe_group(const int32_t *ids, int n_pairs, int n_used, int n_expert,
                      int32_t *grp_expert, int32_t *grp_start, int32_t *grp_count,
                      int32_t *sub_start, int32_t *slot_of_pair, int32_t *pair_idx,

@@ -420,6 +420,7 @@ struct BatchParams {
     int single_count;            // grp_expert == nullptr: one group, expert 0, this many tokens
     const GroupItem *sub_info;   // optional: each chunk's / twin's record
     const GroupItem *twin_info;  //   (launch_moe_group), else a binary search
+    const GroupItem *wide_info;  // units of up to WIDE_CHUNKS chunks (q6k_mv_batched_wide)
     // optional second matrix of the same shape on the same activations (gate
     // and up in one launch): items from items_per_mat on use w2 / y2
     const uint8_t *w2;
@@ -1504,6 +1505,155 @@ __global__ __launch_bounds__(256) void q6k_mv_batched_fast_staged(BatchParams pk
     }
 }
 
+// The grouped kernel for experts with many tokens: a workgroup takes up to
+// WIDE_CHUNKS 16-token chunks of one expert (a unit) against 8 waves of one
+// 16-row tile each. A wave folds a block of its tile into digits once (32
+// registers) and runs them against every chunk, whose planes all 8 waves read
+// from LDS (double-buffered direct global-to-LDS copies, one barrier per
+// block), so the fold costs a quarter of what it costs a twin and a plane is
+// read from L2 once per 128 rows. PAIR: waves 0..3 and 4..7 take the same rows
+// of gate and up, and the output is silu(gate) * up (up through LDS).
+// 128 registers: four waves a SIMD, so that folds, MFMAs and float epilogues
+// of different waves overlap (two tiles a wave halve the LDS reads but leave
+// two waves a SIMD: the same at 2000 tokens, 2-3% slower at 100-512; 16 chunks
+// a unit leave one workgroup a CU: 453 us instead of 367 at 2000).
+// At 2000 tokens the copies and stores alone take 65% of the time and the
+// arithmetic alone 65%; gate + up 185 us, down 100 (traced 350 and 190 as twins).
+// A unit's workgroups run on one XCD (workgroup i on XCD i % 8), which then
+// reads the unit's planes and each weight once.
+constexpr int WIDE_CHUNKS = GROUP_WIDE_CHUNKS;
+
+template <bool PAIR>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void q6k_mv_batched_wide(
+    BatchParams p, int row_groups) {
+    __shared__ float ds[WIDE_MAX_BLOCKS][WIDE_CHUNKS * 16];
+    __shared__ uint64_t tab[32];
+    const int lane = threadIdx.x & 63, n = lane & 15, s = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = blockIdx.x / 8;
+    const int unit = (q / row_groups) * 8 + blockIdx.x % 8, rg = q % row_groups;
+    const GroupItem it = p.wide_info[unit];
+    if (it.expert < 0) return;
+    const int nc = it.twin2;
+    const int t = PAIR ? rg * 4 + (wave & 3) : rg * 8 + wave;
+    const bool live = t < p.tiles;  // (a wave past the last tile works on the last one and stores nothing)
+    const uint8_t *seg = (PAIR && wave >= 4 ? p.w2 : p.w) + (size_t)it.expert * p.expert_stride +
+                         (size_t)min(t, p.tiles - 1) * p.blocks * SEG_BYTES;
+    const size_t chunk_q = (size_t)p.blocks * CHUNK_BLOCK_BYTES, chunk_d = (size_t)p.blocks * CHUNK_TOKENS;
+    int8_t *lds = (int8_t *)g_act_lds;  // [2][WIDE_CHUNKS][4096]
+    // plane wave % 4 of every second chunk of block b, 16 bytes a lane
+    const int u0 = wave >> 2, po = 1024 * (wave & 3);
+    const int8_t *gq = p.act_q + (size_t)(it.sub + u0) * chunk_q + po + 16 * lane;
+    auto stage = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < WIDE_CHUNKS; u += 2)
+            if (u + u0 < nc)
+                __builtin_amdgcn_global_load_lds(
+                    (const void *)(gq + u * chunk_q + (size_t)b * CHUNK_BLOCK_BYTES),
+                    (lds_ptr)(lds + ((b & 1) * WIDE_CHUNKS + u + u0) * CHUNK_BLOCK_BYTES + po), 16, 0, 0);
+    };
+    struct W {
+        uint4 q0, q1, q2;
+        uint32_t scw;
+        uint2 dw;
+    } w;
+    auto wload = [&](int b) {
+        const uint8_t *sg = seg + (size_t)b * SEG_BYTES;
+        w.q0 = *(const uint4 *)(sg + 16 * lane);
+        w.q1 = *(const uint4 *)(sg + SEG_PART + 16 * lane);
+        w.q2 = *(const uint4 *)(sg + 2 * SEG_PART + 16 * lane);
+        w.scw = *(const uint32_t *)(sg + SEG_SC + 4 * lane);
+        w.dw = *(const uint2 *)(sg + SEG_D + 8 * s);  // f16 d of rows 4s..4s+3
+    };
+    stage(0);
+    wload(0);
+    // every block's scales of the unit's tokens
+    for (int i = threadIdx.x; i < nc * (int)chunk_d; i += 512) {
+        const int u = i / (int)chunk_d, r = i % (int)chunk_d;
+        ds[r / 16][u * 16 + r % 16] = p.act_d[(size_t)it.sub * chunk_d + i];
+    }
+    if (PAIR && wave == 0) expf_ref_tab_fill(tab);
+    float acc[WIDE_CHUNKS][4];
+#pragma unroll
+    for (int u = 0; u < WIDE_CHUNKS; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[u][v] = 0.0f;
+    for (int b = 0; b < p.blocks; ++b) {
+        v4i lo[4], hi[4];
+        {
+            const uint32_t nib[8] = {w.q0.x, w.q0.y, w.q0.z, w.q0.w, w.q1.x, w.q1.y, w.q1.z, w.q1.w};
+            const uint32_t hb[4] = {w.q2.x, w.q2.y, w.q2.z, w.q2.w};
+            const FoldScales fs = fold_scales(w.scw);
+#pragma unroll
+            for (int P = 0; P < 4; ++P) fold_pair(nib, hb, P, fs, lo[P], hi[P]);
+        }
+        const float d4[4] = {f16_bits_to_f32((uint16_t)(w.dw.x & 0xFFFF)), f16_bits_to_f32((uint16_t)(w.dw.x >> 16)),
+                             f16_bits_to_f32((uint16_t)(w.dw.y & 0xFFFF)), f16_bits_to_f32((uint16_t)(w.dw.y >> 16))};
+        // this wave's pieces of block b have landed (with its weights, used
+        // above); past the barrier everyone's have, and the other buffer is read
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (b + 1 < p.blocks) {
+            stage(b + 1);
+            wload(b + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const int8_t *aq = lds + (b & 1) * WIDE_CHUNKS * CHUNK_BLOCK_BYTES + 16 * lane;
+#pragma unroll
+        for (int u = 0; u < WIDE_CHUNKS; ++u) {
+            if (u < nc) {
+                const v4i zero = {0, 0, 0, 0};
+                v4i ah = zero, al = zero;
+#pragma unroll
+                for (int P = 0; P < 4; ++P) {
+                    const v4i av = *(const v4i *)(aq + u * CHUNK_BLOCK_BYTES + 1024 * P);
+                    ah = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi[P], av, ah, 0, 0, 0);
+                    al = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo[P], av, al, 0, 0, 0);
+                }
+                const float adb = ds[b][u * 16 + n];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int aux = ah[v] * 256 + al[v];
+                    acc[u][v] = __builtin_fmaf(d4[v] * adb, (float)aux, acc[u][v]);
+                }
+            }
+        }
+    }
+    if constexpr (PAIR) {
+        // up's sums to gate's waves, in the buffers of the planes
+        __syncthreads();
+        float4 *ex = (float4 *)g_act_lds + (wave & 3) * WIDE_CHUNKS * 64 + lane;
+        if (wave >= 4) {
+#pragma unroll
+            for (int u = 0; u < WIDE_CHUNKS; ++u)
+                if (u < nc) ex[u * 64] = make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
+        }
+        __syncthreads();
+        if (wave >= 4) return;
+#pragma unroll
+        for (int u = 0; u < WIDE_CHUNKS; ++u)
+            if (u < nc) {
+                const float4 up = ex[u * 64];
+                acc[u][0] = silu_ref(acc[u][0], tab) * up.x;
+                acc[u][1] = silu_ref(acc[u][1], tab) * up.y;
+                acc[u][2] = silu_ref(acc[u][2], tab) * up.z;
+                acc[u][3] = silu_ref(acc[u][3], tab) * up.w;
+            }
+    }
+    if (!live) return;
+#pragma unroll
+    for (int u = 0; u < WIDE_CHUNKS; ++u) {
+        const int tok = 16 * (it.st + u) + n;
+        if (u < nc && tok < it.count) {
+            const int pos = it.start + tok;
+            const int orow = p.pair_out ? p.pair_out[pos] : pos;
+            // (p.rows % 16 == 0, rows 16-byte aligned: checked at launch)
+            *(float4 *)(p.y + (size_t)orow * p.ldy + t * TILE_ROWS + 4 * s) =
+                make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
+        }
+    }
+}
+
 // ---- LM head: certified arg-max over REDUCTION-tolerance logits -------------
 //
 // The fast batched kernel's logit F_r of row r and the reference's E_r are two
@@ -2005,6 +2155,7 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
     p.y2 = y2;
     p.sub_info = group_tables ? (const GroupItem *)(sub_start + group_items_offset(n_groups)) : nullptr;
     p.twin_info = group_tables ? p.sub_info + max_chunks : nullptr;
+    p.wide_info = group_tables ? p.twin_info + max_chunks : nullptr;
     p.single_count = n_groups;  // only read when grp_expert == nullptr
     p.w = (const uint8_t *)w;
     p.expert_stride = expert_stride;
@@ -2076,6 +2227,33 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
     const long all = w2 ? 2 * items : items;
     if (!grp_expert) return launch_one_group(p, all, st);
     hipLaunchKernelGGL(q6k_mv_batched, dim3((unsigned)((all + 3) / 4)), dim3(256), 0, st, p);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+bool q6k_wide_fits(int rows, int blocks) { return rows % TILE_ROWS == 0 && blocks <= WIDE_MAX_BLOCKS; }
+
+int launch_q6k_mv_batched_wide(const void *w, const void *w2, size_t expert_stride,
+                               const int32_t *sub_start, const int32_t *pair_out,
+                               const int8_t *act_q, const float *act_d, float *y, int rows,
+                               int blocks, int n_groups, int max_chunks, hipStream_t st) {
+    if (!q6k_wide_fits(rows, blocks) || (uintptr_t)y % 16 || max_chunks <= 0) return -1;
+    BatchParams p = {};
+    p.w = (const uint8_t *)w;
+    p.w2 = (const uint8_t *)w2;
+    p.expert_stride = expert_stride;
+    p.wide_info = (const GroupItem *)(sub_start + group_items_offset(n_groups)) + 2 * (size_t)max_chunks;
+    p.pair_out = pair_out;
+    p.act_q = act_q;
+    p.act_d = act_d;
+    p.y = y;
+    p.ldy = p.rows = rows;
+    p.tiles = rows / TILE_ROWS;
+    p.blocks = blocks;
+    const int row_groups = w2 ? (p.tiles + 3) / 4 : (p.tiles + 7) / 8;
+    const int units = group_wide_units(n_groups, max_chunks);
+    constexpr size_t lds = 2 * WIDE_CHUNKS * CHUNK_BLOCK_BYTES;
+    if (w2) hipLaunchKernelGGL(q6k_mv_batched_wide<true>, dim3(units * row_groups), dim3(512), lds, st, p, row_groups);
+    else hipLaunchKernelGGL(q6k_mv_batched_wide<false>, dim3(units * row_groups), dim3(512), lds, st, p, row_groups);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
