@@ -620,8 +620,7 @@ __device__ __forceinline__ void tile_block(const TileRegs &r, const float (&adb)
 // activations (local chunk numbers st0.. inside the group of `cnt` pairs
 // starting at sorted position `start`). The weight codes are unpacked and
 // folded once per class and feed the MFMAs of all NC chunks, so a second
-// chunk costs only its MFMAs and its float epilogue. Each chunk's class plane
-// of a block is one contiguous 512-byte load for the wave.
+// chunk costs only its MFMAs and its float epilogue.
 template <int NC, bool PF = false>
 __device__ __forceinline__ void batched_tile(const BatchParams &p, int lane, int t, int sub0,
                                              int st0, int cnt, int start, int expert) {
