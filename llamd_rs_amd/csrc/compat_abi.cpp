@@ -443,7 +443,9 @@ void attend(const float *q, const float *kc, const float *vc, float *out, int n_
     // what one sequence can hold: all of the kernels' range when the position
     // is on the device and only this cache is read, else its slice
     const int cap = !pos ? n_kv : nseq == 1 ? attend_max_kv() : max_kv;
-    if (attend_split_fits(n_head, n_head_kv, hd, cap)) {
+    // (out over q: attend_decode's one workgroup per head has read q before it
+    // writes; a head's two workgroups in the split form have not)
+    if (out != q && attend_split_fits(n_head, n_head_kv, hd, cap)) {
         std::lock_guard<std::mutex> lk(g_smu);
         float *scores = (float *)scratch(attend_split_scores(n_head, cap, nseq) * 4);
         if (!scores) return fwd_refused();

@@ -90,6 +90,32 @@ def test_batched_attention_past_its_slice(gpu):
     assert np.isnan(got[1:]).all()
 
 
+@pytest.mark.parametrize("n_kv", [1, 40, 64, 130, 400])
+def test_attention_over_its_own_input(gpu, n_kv):
+    """out over q, one sequence and two: the bits of a call with a buffer of its own."""
+    n_head, n_head_kv, hd, max_kv = 32, 4, 128, 512
+    kv_dim = n_head_kv * hd
+    q = (H.sample(2 * n_head * hd, 96) * 3).astype(np.float32).reshape(2, -1)
+    kc = H.sample(2 * max_kv * kv_dim, 97).reshape(2, max_kv, kv_dim)
+    vc = H.sample(2 * max_kv * kv_dim, 98).reshape(2, max_kv, kv_dim)
+    L = gpu.lib()
+    K, V = gpu.DeviceBuffer.from_array(kc), gpu.DeviceBuffer.from_array(vc)
+    M = gpu.DeviceBuffer.from_array(np.array([[0, n_kv - 1]] * 2, np.int32))
+    want = [O.attend(q[s], kc[s, :n_kv], vc[s, :n_kv], n_kv, n_head, n_head_kv, hd) for s in range(2)]
+    for call in ("fixed", "meta", "batch"):
+        Q = gpu.DeviceBuffer.from_array(q)
+        if call == "fixed":
+            L.llamd_fwd_attention(Q.ptr, K.ptr, V.ptr, Q.ptr, None, n_head, n_head_kv, hd, n_kv)
+        elif call == "meta":
+            L.llamd_fwd_attention_meta(Q.ptr, K.ptr, V.ptr, Q.ptr, None, n_head, n_head_kv, hd, M.ptr, max_kv)
+        else:
+            L.llamd_b_attention(Q.ptr, K.ptr, V.ptr, Q.ptr, None, n_head, n_head_kv, hd, max_kv, M.ptr, 2)
+        assert L.llamd_fwd_sync() == 0 and L.llamd_fwd_last_error() == 0
+        got = Q.download(np.empty_like(q))
+        assert bits_equal(got[0], want[0]), call
+        assert bits_equal(got[1], want[1] if call == "batch" else q[1]), call
+
+
 @pytest.mark.parametrize("n_kv", [50, 400])
 def test_attention_non_finite_and_lowest_logits(gpu, n_kv):
     """Keys that make a logit -inf, NaN or hugely negative, and a V row of
