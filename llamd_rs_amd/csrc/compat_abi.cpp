@@ -117,6 +117,7 @@ void *scratch(size_t bytes) {
     const size_t cap = std::max<size_t>({bytes, 2 * g_scr_cap, (size_t)4 << 20});
     void *p = nullptr;
     if (hipMalloc(&p, cap) != hipSuccess) {
+        (void)hipGetLastError();  // or the next launch's check would find it
         set_error("scratch: hipMalloc of %zu bytes", cap);
         return nullptr;
     }
@@ -446,13 +447,18 @@ void attend(const float *q, const float *kc, const float *vc, float *out, int n_
     // (out over q: attend_decode's one workgroup per head has read q before it
     // writes; a head's two workgroups in the split form have not)
     if (out != q && attend_split_fits(n_head, n_head_kv, hd, cap)) {
-        std::lock_guard<std::mutex> lk(g_smu);
-        float *scores = (float *)scratch(attend_split_scores(n_head, cap, nseq) * 4);
-        if (!scores) return fwd_refused();
-        if (launch_attend_split(q, kc, vc, pos, n_head, n_head_kv, hd, scale, cap, scores, out, S(), nseq,
-                                n_kv, pos_stride, (size_t)max_kv * n_head_kv * hd, pos ? max_kv : n_kv))
-            REFUSE("attention: launch");
-        return;
+        const int expect = pos ? max_kv : n_kv;
+        const size_t need = attend_split_scores(n_head, cap, nseq, expect) * 4;
+        std::unique_lock<std::mutex> lk(g_smu, std::defer_lock);
+        if (need) lk.lock();
+        float *scores = need ? (float *)scratch(need) : nullptr;
+        if (scores || !need) {
+            if (launch_attend_split(q, kc, vc, pos, n_head, n_head_kv, hd, scale, cap, scores, out, S(), nseq,
+                                    n_kv, pos_stride, (size_t)max_kv * n_head_kv * hd, expect))
+                REFUSE("attention: launch");
+            return;
+        }
+        // no memory for the logits: attend_decode keeps them in LDS
     }
     if (launch_attend_decode(q, kc, vc, pos, n_head, n_head_kv, hd, scale, out, S(), nseq, n_kv,
                              pos_stride, (size_t)max_kv * n_head_kv * hd))

@@ -953,14 +953,23 @@ bool attend_split_fits(int n_head, int n_head_kv, int hd, int max_kv) {
            max_kv <= ATT_MAX_KV;
 }
 
-size_t attend_split_scores(int n_head, int cap, int nseq) { return (size_t)nseq * n_head * cap; }
+namespace {
+// The most positions that the one-launch form is chosen for (launch_attend_split).
+constexpr int ATT_ONE_LAUNCH = 256;
+int split_expect(int cap, int expect) { return expect <= 0 || expect > cap ? cap : expect; }
+}  // namespace
+
+size_t attend_split_scores(int n_head, int cap, int nseq, int expect) {
+    return split_expect(cap, expect) <= ATT_ONE_LAUNCH ? 0 : (size_t)nseq * n_head * cap;
+}
 
 int launch_attend_split(const float *q, const float *kc, const float *vc, const int32_t *pos,
                         int n_head, int n_head_kv, int hd, float scale, int cap, float *scores,
                         float *out, hipStream_t st, int nseq, int n_kv_fixed, int pos_stride,
                         size_t cache_seq_stride, int expect) {
     if (!attend_split_fits(n_head, n_head_kv, hd, cap) || nseq <= 0 || nseq > 65535) return -1;
-    if (expect <= 0 || expect > cap) expect = cap;
+    expect = split_expect(cap, expect);
+    if (!scores && expect > ATT_ONE_LAUNCH) return -1;
     AttArgs a{};
     a.q = q;
     a.kc = kc;
@@ -980,7 +989,7 @@ int launch_attend_split(const float *q, const float *kc, const float *vc, const 
     // (attend_decode alone, then this): 1 sequence of 250 positions 15.2, 13.2;
     // 1000: 49, 16.8; 4100: 278, 34.5; 8192: 544, 56; 13 of up to 1000: 88, 29;
     // 16 of up to 2000: 185, 49; of up to 40: 10.5, 8.9.
-    if (expect <= 256) {
+    if (expect <= ATT_ONE_LAUNCH) {
         // short caches: one launch of small workgroups that form the logits
         // themselves (at 300 positions the second launch already pays)
         a.fuse = cap;

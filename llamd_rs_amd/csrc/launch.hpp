@@ -247,12 +247,12 @@ int launch_attend_fused(const float *q, const float *k, const float *v, const fl
 // the logits by blocks of positions, then the softmax (exact in-order sum) and
 // the in-order weighted V sum per head, into out [nseq][n_head * hd]; the bits
 // of launch_attend_decode. cap: positions that scores (attend_split_scores
-// floats) and the LDS hold per head; a sequence that has more is still
-// attended to, slowly. expect: the most positions a sequence is expected to
-// have (0: cap), which only decides how the work is split. Sequences as in
-// launch_attend_decode.
+// floats; none for the one launch of short caches, scores null) and the LDS
+// hold per head; a sequence that has more is still attended to, slowly.
+// expect: the most positions a sequence is expected to have (0: cap), which
+// only decides how the work is split. Sequences as in launch_attend_decode.
 bool attend_split_fits(int n_head, int n_head_kv, int hd, int max_kv);
-size_t attend_split_scores(int n_head, int cap, int nseq);
+size_t attend_split_scores(int n_head, int cap, int nseq, int expect = 0);
 int launch_attend_split(const float *q, const float *kc, const float *vc, const int32_t *pos,
                         int n_head, int n_head_kv, int hd, float scale, int cap, float *scores,
                         float *out, hipStream_t st, int nseq = 1, int n_kv_fixed = 0,

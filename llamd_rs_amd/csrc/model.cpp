@@ -350,8 +350,8 @@ void *llamd_hip_model_create(void *g, int max_kv) {
     m->tokpos = (int32_t *)dalloc(*m, 16);
     m->next = (int32_t *)dalloc(*m, 16);
     if (m->split_attn) {
-        m->scores = dalloc(*m, llamd::attend_split_scores(m->n_head, max_kv, 1) * 4);
-        if (!m->scores) m->split_attn = false;
+        const size_t need = llamd::attend_split_scores(m->n_head, max_kv, 1) * 4;
+        if (need && !(m->scores = dalloc(*m, need))) m->split_attn = false;
     }
     if (hipHostMalloc((void **)&m->stage, 64, hipHostMallocDefault) != hipSuccess) m->stage = nullptr;
     if (!m->x || !m->xn || !m->ffn_inp || !m->fn || !m->o || !m->q || !m->attn || !m->k || !m->v ||

@@ -90,6 +90,26 @@ def test_batched_attention_past_its_slice(gpu):
     assert np.isnan(got[1:]).all()
 
 
+def test_short_caches_take_no_device_memory(gpu):
+    """4096 sequences of one position in slices of 256: the launch forms the
+    logits itself, so none of the 256 MiB that they would fill is allocated.
+    One position: the output is its V row."""
+    nseq, n_head, n_head_kv, hd, max_kv = 4096, 16, 1, 64, 256
+    q = H.sample(nseq * n_head * hd, 99).reshape(nseq, n_head, hd)
+    v = H.sample(nseq * max_kv * hd, 100).reshape(nseq, max_kv, hd)
+    L = gpu.lib()
+    Q, K, V = (gpu.DeviceBuffer.from_array(a) for a in (q, v, v))
+    M = gpu.DeviceBuffer.from_array(np.zeros((nseq, 2), np.int32))
+    out = gpu.DeviceBuffer(q.nbytes)
+    assert L.llamd_fwd_sync() == 0
+    free = L.llamd_rocm_free_mem()
+    L.llamd_b_attention(Q.ptr, K.ptr, V.ptr, out.ptr, None, n_head, n_head_kv, hd, max_kv, M.ptr, nseq)
+    assert L.llamd_fwd_sync() == 0 and L.llamd_fwd_last_error() == 0
+    assert free - L.llamd_rocm_free_mem() < 64 << 20
+    got = out.download(np.empty_like(q))
+    assert np.array_equal(got, np.broadcast_to(v[:, :1], got.shape))
+
+
 @pytest.mark.parametrize("n_kv", [1, 40, 64, 130, 400])
 def test_attention_over_its_own_input(gpu, n_kv):
     """out over q, one sequence and two: the bits of a call with a buffer of its own."""
