@@ -465,8 +465,10 @@ __global__ __launch_bounds__(512) void attend_fused(
 // four products and add them: other waves load V a few chunks ahead, multiply
 // by the weights and hand chunks of products over in LDS, transposed so that a
 // lane's four next products are one read. What is left is the chain itself, 3.6
-// ns per position, and about 1.2 ns of waiting for the products; a barrier per
-// 32 positions instead of 128 (64 where CUs are shared) costs another 2-4 ns.
+// ns per position, and 1-1.5 ns of waiting for the products; a barrier per
+// 32 positions instead of 128 (64 for all 128 dimensions in one workgroup) costs
+// another 2-4 ns. The last chunk ends with its last 32 positions (one sequence of
+// 20: 8.1, 7.5 us a call; of 150 11.9, 11.0).
 // The same operations in the same order as attend_decode (and the reference,
 // attention.rs:73-125): the same bits.
 constexpr int AS_POS = 64;          // positions per block of attend_scores
@@ -624,7 +626,9 @@ __device__ __forceinline__ void att_beyond_cap(const AttArgs &a, const float *q,
     if (tid < DS) out[tid] = acc;
 }
 
-// e_t summed in order from 0 by one lane, 32 read per step.
+// e_t summed in order from 0 by one lane, 32 read per step. The e_t up to the
+// next multiple of 32 are +0.0, which leaves the sum as it is (it is never
+// -0.0), so the last step needs no terms one by one (20 terms: 0.4 us less).
 __device__ __forceinline__ float att_sum_serial(const float *lg, int n) {
     float sum = 0.0f;
     int t = 0;
@@ -635,7 +639,16 @@ __device__ __forceinline__ float att_sum_serial(const float *lg, int n) {
 #pragma unroll
         for (int j = 0; j < 32; ++j) sum = sum + e[j / 4][j % 4];
     }
-    for (; t < n; ++t) sum = sum + lg[t];
+    if (t < n) {
+        att_f4 e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = *(const att_f4 *)(lg + t + 4 * j);
+#pragma unroll
+        for (int j = 0; j < 32; ++j) {
+            if (j && j % 8 == 0 && t + j >= n) break;
+            sum = sum + e[j / 4][j % 4];
+        }
+    }
     return sum;
 }
 
@@ -695,8 +708,8 @@ __device__ __forceinline__ float att_logits_here(const float *q, const float *kc
 template <int DS, int NP, bool WIDE>
 constexpr int am_threads = WIDE ? 64 * (1 + (NP + 2) / 3 * 3 + (NP - 1) / 3) : DS + 64 * NP;
 // Positions per chunk: one 4 x 4 piece of products per producer thread, or two
-// where several workgroups share the CU (a barrier and a hand-over per 64
-// positions instead of 32).
+// where several workgroups share the CU (a barrier and a hand-over per 128
+// positions of 64 dimensions or 64 of 128, instead of half).
 template <int DS, int NP, bool WIDE>
 constexpr int am_chunk = (WIDE ? 1 : 2) * 1024 * NP / DS;
 
@@ -780,6 +793,7 @@ __global__ __launch_bounds__((am_threads<DS, NP, WIDE>)) void attend_mix(AttArgs
 #pragma unroll
     for (int w = 0; w < NW; ++w) mx = fmaxf(mx, red[w]);
     for (int t = tid; t < n_kv; t += NT) lg[t] = expf_ref_tab(lg[t] - mx, tab);
+    if (tid >= n_kv % 32 && tid < 32 && n_kv % 32) lg[n_kv / 32 * 32 + tid] = 0.0f;  // (att_sum_serial)
     __syncthreads();
     if (n_kv <= ATT_SERIAL) {
         if (tid == 0) inv1 = __fdiv_rn(1.0f, att_sum_serial(lg, n_kv));
@@ -820,24 +834,38 @@ __global__ __launch_bounds__((am_threads<DS, NP, WIDE>)) void attend_mix(AttArgs
     if (folds) {
         __builtin_amdgcn_s_setprio(3);
         float acc = 0.0f;
-        for (int c = 0; c < nc; ++c) {
+        // 32 products ahead of the 32 being added
+        att_f4 p[2][8];
+        const auto read = [&](const float *src, int k) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) p[k & 1][i] = *(const att_f4 *)(src + (8 * k + i) * DS * 4);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        const auto add = [&](int k) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc = acc + p[k & 1][i][e];
+        };
+        // the last chunk ends with its last 32 positions; zeros follow
+        const int left = n_kv - (nc - 1) * CH, full = left > CH - 32 ? nc : nc - 1;
+        for (int c = 0; c < full; ++c) {
             __syncthreads();
             const float *src = buf + (c & 1) * (CH * DS) + tid * 4;
-            // 32 products ahead of the 32 being added
-            att_f4 p[2][8];
-            const auto read = [&](int k) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) p[k & 1][i] = *(const att_f4 *)(src + (8 * k + i) * DS * 4);
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            read(0);
+            read(src, 0);
 #pragma unroll
             for (int k = 0; k < CH / 32; ++k) {
-                if (k + 1 < CH / 32) read(k + 1);
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc = acc + p[k & 1][i][e];
+                if (k + 1 < CH / 32) read(src, k + 1);
+                add(k);
+            }
+        }
+        if (full < nc) {
+            __syncthreads();
+            const float *src = buf + (full & 1) * (CH * DS) + tid * 4;
+#pragma unroll 1
+            for (int t = 0; t < left; t += 32, src += 32 * DS) {
+                read(src, 0);
+                add(0);
             }
         }
         out[(tid % D4) * 4 + tid / D4] = acc;
@@ -998,9 +1026,15 @@ int launch_attend_split(const float *q, const float *kc, const float *vc, const 
                             : launch_mix<128, 128, 4, false, 1>(a, nseq, st);
     }
     a.fuse = 64;
-    const int blocks = (expect + AS_POS - 1) / AS_POS;
-    const int share = 2048 / (n_head_kv * nseq);
-    a.grid_x = blocks < share ? blocks : share > 0 ? share : 1;
+    // 16 waves a CU (at most 2048 workgroups), which take several blocks each
+    // where there are more: a slice may be mostly empty, and each workgroup that
+    // finds nothing to do still costs its launch (us with 2048 workgroups of 8
+    // waves, then 512: 16 sequences of 100 positions in slices of 2048 19.7, 13.3;
+    // of 2000 54, 51; 1 of 8192 56, 56. With 256, 16 of 4096 147 against 135).
+    // Slices of up to 1024 may have 32 a CU, one round (13 of 1000 28.8, 29.3 with 512).
+    const int blocks = (expect + AS_POS - 1) / AS_POS, pairs = n_head_kv * nseq;
+    const int most = std::min(2048, (blocks <= 16 ? 8192 : 4096) / (n_head / n_head_kv));
+    a.grid_x = std::min(blocks, (most + pairs - 1) / pairs);
     const dim3 grid(a.grid_x, n_head_kv, nseq), block(64 * (n_head / n_head_kv));
     if (hd == 128) hipLaunchKernelGGL(attend_scores<128>, grid, block, 0, st, a);
     else hipLaunchKernelGGL(attend_scores<64>, grid, block, 0, st, a);
@@ -1008,14 +1042,17 @@ int launch_attend_split(const float *q, const float *kc, const float *vc, const 
     // a CU to a workgroup while every one finds its own (1..4 sequences of
     // 1000: 16.8-18.3 us, 17.2-18.7 with the small workgroups); then small
     // workgroups on 64 dimensions up to one per CU and dimension half (8 of
-    // 500: 16.9, 18.9 with all 128 dimensions), then on all (13 of 1000: 28.9,
-    // 36 with 64)
+    // 500: 16.9, 18.9 with all 128 dimensions; of 2000 34, 41) where a CU's LDS
+    // holds two of them, then on all (13 of 1000: 28.9, 36 with 64; 8 in slices
+    // of 8192, with 64 and with 128 dimensions: 20 positions 13.4, 8.9; 500 24.5,
+    // 19.5; 8000 162, 129)
     if (hd == 64)
         return heads <= 128 ? launch_mix<64, 64, 8, true, 1>(a, nseq, st)
                             : launch_mix<64, 64, 4, false, 1>(a, nseq, st);
     if (heads <= 128) return launch_mix<128, 64, 8, true, 1>(a, nseq, st);
-    return heads <= 256 ? launch_mix<128, 64, 4, false, 1>(a, nseq, st)
-                        : launch_mix<128, 128, 4, false, 1>(a, nseq, st);
+    const bool two = 2 * (split_lds(cap, 128, 64, am_chunk<64, 4, false>, 1) + sizeof(ExactSumLds) + 1024) <= 160 * 1024;
+    return heads <= 256 && two ? launch_mix<128, 64, 4, false, 1>(a, nseq, st)
+                               : launch_mix<128, 128, 4, false, 1>(a, nseq, st);
 }
 
 int launch_attend_decode(const float *q, const float *kc, const float *vc, const int32_t *pos,

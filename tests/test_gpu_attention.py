@@ -1,8 +1,10 @@
 """The attention entry points against the oracle's in-order composition, bit
 for bit, where the split over positions, heads and dimensions can go wrong:
-blocks of 64 positions, chunks of 32 and 64 positions, the pieces of the exact
-sum (6656 to 8192 terms), both sides of the fused logits, ragged batches, a
-position beyond a sequence's slice and the values that softmax ignores."""
+blocks of 64 positions, chunks of 64 and 128 positions and the 32 that the last
+one ends with, the pieces of the exact sum (2560, 3072 and 6144 terms on
+workgroups of 320, 384 and 768 threads), both sides of the fused logits, ragged
+batches, a position beyond a sequence's slice and the values that softmax
+ignores."""
 import numpy as np
 import pytest
 
@@ -32,9 +34,9 @@ def run_one(gpu, q, kc, vc, n_head, n_head_kv, hd, n_kv, max_kv=None):
 
 
 @pytest.mark.parametrize("n_head,n_head_kv,hd,lengths", [
-    (32, 4, 128, (1, 31, 64, 65, 256, 257, 1000, 4100)),
-    (8, 1, 128, (6656, 6657, 8193, 16384)),
-    (12, 12, 64, (1, 63, 64, 129, 300, 2051)),
+    (32, 4, 128, (1, 8, 20, 31, 64, 65, 96, 97, 129, 160, 161, 256, 257, 352, 1000, 4100)),
+    (8, 1, 128, (6144, 6145, 6657, 8193, 16384)),
+    (12, 12, 64, (1, 63, 64, 97, 129, 300, 2051)),
     (16, 1, 64, (65, 700)),
     (4, 2, 32, (40, 300)), (34, 2, 128, (130,))])   # these two on the general kernel
 def test_attention_bit_exact(gpu, n_head, n_head_kv, hd, lengths):
@@ -52,7 +54,8 @@ def test_attention_bit_exact(gpu, n_head, n_head_kv, hd, lengths):
 
 
 @pytest.mark.parametrize("nseq,n_head,n_head_kv,hd,max_kv", [
-    (3, 32, 4, 128, 300), (13, 32, 4, 128, 200), (16, 12, 12, 64, 160), (2, 8, 8, 128, 700)])
+    (3, 32, 4, 128, 300), (13, 32, 4, 128, 200), (16, 12, 12, 64, 160), (2, 8, 8, 128, 700),
+    (13, 32, 4, 128, 500), (16, 12, 12, 64, 420), (7, 32, 4, 128, 700)])
 def test_batched_attention_ragged_bit_exact(gpu, nseq, n_head, n_head_kv, hd, max_kv):
     kv_dim = n_head_kv * hd
     q = (H.sample(nseq * n_head * hd, 84) * 3).astype(np.float32).reshape(nseq, -1)
@@ -60,6 +63,23 @@ def test_batched_attention_ragged_bit_exact(gpu, nseq, n_head, n_head_kv, hd, ma
     vc = H.sample(nseq * max_kv * kv_dim, 86).reshape(nseq, max_kv, kv_dim)
     lengths = [(max_kv * (s + 1) // nseq) for s in range(nseq)]
     lengths[0] = 1
+    check_batch(gpu, q, kc, vc, n_head, n_head_kv, hd, lengths)
+
+
+@pytest.mark.parametrize("max_kv,lengths", [(2600, (1, 63, 65, 2560, 2561)), (3400, (31, 33, 95, 129, 3072, 3073))])
+def test_batched_attention_sum_pieces(gpu, max_kv, lengths):
+    """129..256 heads: on 64 dimensions each where a CU's LDS holds two
+    workgroups (up to 3300 positions), else on all 128."""
+    n_head, n_head_kv, hd, nseq = 32, 4, 128, len(lengths)
+    kv_dim = n_head_kv * hd
+    q = (H.sample(nseq * n_head * hd, 84) * 3).astype(np.float32).reshape(nseq, -1)
+    kc = H.sample(nseq * max_kv * kv_dim, 85).reshape(nseq, max_kv, kv_dim)
+    vc = H.sample(nseq * max_kv * kv_dim, 86).reshape(nseq, max_kv, kv_dim)
+    check_batch(gpu, q, kc, vc, n_head, n_head_kv, hd, lengths)
+
+
+def check_batch(gpu, q, kc, vc, n_head, n_head_kv, hd, lengths):
+    nseq, max_kv = kc.shape[:2]
     meta = np.array([[7, n - 1] for n in lengths], np.int32)
     L = gpu.lib()
     Q, K, V, M = (gpu.DeviceBuffer.from_array(a) for a in (q, kc, vc, meta))
