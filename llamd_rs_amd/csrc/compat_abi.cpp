@@ -446,7 +446,7 @@ void attend(const float *q, const float *kc, const float *vc, float *out, int n_
     const int cap = !pos ? n_kv : nseq == 1 ? attend_max_kv() : max_kv;
     // (out over q: attend_decode's one workgroup per head has read q before it
     // writes; a head's two workgroups in the split form have not)
-    if (out != q && attend_split_fits(n_head, n_head_kv, hd, cap)) {
+    if (out != q && nseq <= 65535 && attend_split_fits(n_head, n_head_kv, hd, cap)) {
         const int expect = pos ? max_kv : n_kv;
         const size_t need = attend_split_scores(n_head, cap, nseq, expect) * 4;
         std::unique_lock<std::mutex> lk(g_smu, std::defer_lock);

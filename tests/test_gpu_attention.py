@@ -91,6 +91,20 @@ def check_batch(gpu, q, kc, vc, n_head, n_head_kv, hd, lengths):
         assert bits_equal(got[s], O.attend(q[s], kc[s, :n], vc[s, :n], n, n_head, n_head_kv, hd)), (s, n)
 
 
+def test_batched_attention_more_sequences_than_a_grid_dimension(gpu):
+    """66000 sequences of one position: the output is the V row."""
+    nseq, hd = 66000, 64
+    q = H.sample(nseq * hd, 101).reshape(nseq, hd)
+    v = H.sample(nseq * hd, 102).reshape(nseq, hd)
+    L = gpu.lib()
+    Q, V = (gpu.DeviceBuffer.from_array(a) for a in (q, v))
+    M = gpu.DeviceBuffer.from_array(np.zeros((nseq, 2), np.int32))
+    out = gpu.DeviceBuffer(q.nbytes)
+    L.llamd_b_attention(Q.ptr, V.ptr, V.ptr, out.ptr, None, 1, 1, hd, 1, M.ptr, nseq)
+    assert L.llamd_fwd_sync() == 0 and L.llamd_fwd_last_error() == 0
+    assert np.array_equal(out.download(np.empty_like(q)), v)
+
+
 def test_batched_attention_past_its_slice(gpu):
     """A sequence whose position lies past max_kv is attended to over the rows
     that follow its slice's start, as before; one out of range gives NaN."""
