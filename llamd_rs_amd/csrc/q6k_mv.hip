@@ -1343,18 +1343,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // The same by chunks on one group of tokens (LM head of 151936 rows, 16
 // sequences: 75.7 -> 70.3 us a call; of 32003: 22.4 -> 20.9; QKV of 96 tokens
 // 22.4 -> 21.0, of 512 61.7, 61.8; the whole chunk in LDS before the first
-// block: 73.9, 23.2).
+// block: 73.9, 23.2). Items count staged_slots(tiles) tiles to a chunk, so that a
+// workgroup's four share their chunk; the waves past the last tile only stage
+// (8200 rows, 40 sequences: 16.8 us; 17.8 by a wave per item, which reads its
+// planes from L2 by itself).
+__host__ __device__ constexpr int staged_slots(int tiles) { return (tiles + 3) & ~3; }
+
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void q6k_mv_batched_staged(BatchParams pk) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     BatchParams p;
     const int item = batch_item(pk, p);
-    // the grid's rounding to whole workgroups: those waves only stage
-    const bool live = item < p.items_per_mat;
-    const int chunk = live ? item / p.tiles : 0;
+    const int chunk = item / staged_slots(p.tiles), t = item % staged_slots(p.tiles);
     if (CHUNK_TOKENS * chunk >= p.single_count) return;
-    const GroupItem it = {0, chunk, chunk, live ? p.single_count : 0, 0, 0, 0, 0};
-    exact_tile_staged<1, true>(p, it, lane, wave, live ? item % p.tiles : 0);
+    const GroupItem it = {0, chunk, chunk, t < p.tiles ? p.single_count : 0, 0, 0, 0, 0};
+    exact_tile_staged<1, true>(p, it, lane, wave, min(t, p.tiles - 1));
 }
 
 // The same by chunks, for calls that leave most experts a token or two.
@@ -2120,19 +2123,26 @@ int launch_q6k_mv_routed(const void *w, const void *w_b, size_t expert_stride,
 }
 
 namespace {
-// The exact kernels on one group of tokens, items = tiles x chunks in all.
-int launch_one_group(const BatchParams &p, long items, hipStream_t st) {
-    const dim3 grid((unsigned)((items + 3) / 4));
-    // the 4 tiles of a workgroup share a chunk
-    bool even = p.tiles % 4 == 0;
-    for (int i = 1; i < p.n_segs; ++i) even = even && p.segs[i].tiles % 4 == 0;
+// The exact kernels on one group of tokens in `chunks` chunks, items = tiles x
+// chunks in all.
+int launch_one_group(BatchParams &p, int chunks, long items, hipStream_t st) {
     // half a wave per SIMD or less (us per call with the norm and the quants, a
     // wave per item -> four: 320 items 15.9 -> 14.4, 640 16.3 -> 16.8)
-    if (items <= 512 && !p.amax_v)
+    if (items <= 512 && !p.amax_v) {
         hipLaunchKernelGGL(q6k_mv_batched_classes, dim3((unsigned)items), dim3(256), 0, st, p);
-    else if (p.single_count <= CHUNK_TOKENS || even)
-        hipLaunchKernelGGL(q6k_mv_batched_staged, grid, dim3(256), 2 * CHUNK_BLOCK_BYTES, st, p);
-    else hipLaunchKernelGGL(q6k_mv_batched, grid, dim3(256), 0, st, p);
+        return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
+    long slots = 0;
+    if (p.n_segs > 0) {
+        for (int i = 0; i < p.n_segs; ++i) {
+            p.segs[i].first = (int)slots;
+            slots += p.segs[i].items = staged_slots(p.segs[i].tiles) * chunks;
+        }
+    } else {
+        p.items_per_mat = staged_slots(p.tiles) * chunks;
+        slots = p.w2 ? 2L * p.items_per_mat : p.items_per_mat;
+    }
+    hipLaunchKernelGGL(q6k_mv_batched_staged, dim3((unsigned)(slots / 4)), dim3(256), 2 * CHUNK_BLOCK_BYTES, st, p);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 }  // namespace
@@ -2224,7 +2234,7 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
     if (items <= 0) return 0;
     p.items_per_mat = (int)items;
     const long all = w2 ? 2 * items : items;
-    if (!grp_expert) return launch_one_group(p, all, st);
+    if (!grp_expert) return launch_one_group(p, max_chunks, all, st);
     hipLaunchKernelGGL(q6k_mv_batched, dim3((unsigned)((all + 3) / 4)), dim3(256), 0, st, p);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -2283,7 +2293,7 @@ int launch_q6k_mv_batched_x3(const void *const w[3], float *const y[3], const in
     p.act_d = act_d;
     p.blocks = blocks;
     p.single_count = nseq;  // one group (expert 0) of nseq tokens
-    return launch_one_group(p, first, st);
+    return launch_one_group(p, chunks, first, st);
 }
 
 int launch_q6k_down_combine(const void *w, size_t expert_stride, const int32_t *ids,

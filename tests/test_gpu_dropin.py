@@ -311,6 +311,21 @@ def test_batched_matvecs_exact(gpu, nseq):
                       np.concatenate([O.matvec_q6k_act(w0, 64, k, a) for a in qa]))
 
 
+@pytest.mark.parametrize("rows,nseq", [((4104, 1040, 2072), 20), ((8200, 3, 64), 16), ((5160, 5160, 24), 33)])
+def test_batched_x3_of_uneven_rows_exact(gpu, rows, nseq):
+    """Three matrices of many tiles, none a multiple of four, on one chunk and on more."""
+    blocks = 2
+    ws = [H.weights(r, blocks, 93 + i) for i, r in enumerate(rows)]
+    qa, q, d = acts(nseq, blocks, 110)
+    W = [dev(gpu, w) for w in ws]
+    Q, D = dev(gpu, q), dev(gpu, d)
+    o = [gpu.DeviceBuffer(r * nseq * 4) for r in rows]
+    L().llamd_b_matvec_x3(*(w.ptr for w in W), Q.ptr, D.ptr, *(b.ptr for b in o), blocks, *rows, nseq)
+    sync()
+    for w, r, b in zip(ws, rows, o):
+        assert bits_equal(down(b, r * nseq), np.concatenate([O.matvec_q6k_act(w, r, blocks * QK_K, a) for a in qa])), r
+
+
 @pytest.mark.parametrize("nseq", [1, 3, 8])
 def test_batched_expert_matvecs_exact(gpu, nseq):
     rows, blocks, n_expert, n_used = 256, 8, 8, 4

@@ -73,7 +73,8 @@ def test_grouped_prompt_lengths(gpu, n_tok, n_used):
 
 
 @pytest.mark.parametrize("rows,k,nseq", [(40, 256, 2), (8192, 768, 16), (8197, 512, 1 + 16), (8197, 1280, 16),
-                                         (8256, 512, 16), (8256, 768, 33), (2112, 256, 64)])
+                                         (8256, 512, 16), (8256, 768, 33), (2112, 256, 64),
+                                         (2072, 512, 81), (8216, 256, 40), (8232, 512, 33)])
 def test_one_group_kernels(gpu, rows, k, nseq):
     """One group of tokens on few tiles (classes split over waves), on many
     (planes staged), with a last workgroup that is part empty, and on tiles and
