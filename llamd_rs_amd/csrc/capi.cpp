@@ -1063,8 +1063,17 @@ namespace {
 // per expert on. Measured per call (us, twins staged in LDS -> wide units; 128
 // experts, top 8): 24 tokens 105 -> 106, 45 101 -> 101, 100 124 -> 124, 200
 // 141 -> 132, 512 201..205 -> 161..182, 1000 309 -> 249, 2000 538 -> 367.
+// An expert makes moe_wide_groups workgroups or more; below 512 for all experts,
+// the twins fill the chip better (us, twins -> wide units: 16 experts of 768 x
+// 2048, top 2, 190 tokens 41 -> 42, with skewed routing 40 -> 55; 4 of 2048 x 512,
+// 400 tokens 38 -> 52; at 512, 32 of 1536 x 2048, top 4, 256 tokens 100 -> 81,
+// skewed 97 -> 97).
+int moe_wide_groups(const MoeLayer *m) {
+    return std::min(q6k_wide_groups(m->n_ff, true), q6k_wide_groups(m->n_embd, false));
+}
 bool moe_wide(const MoeLayer *m, int n_pairs) {
-    return n_pairs / 8 >= m->n_expert && q6k_wide_fits(m->n_ff, m->be) && q6k_wide_fits(m->n_embd, m->bf);
+    return n_pairs / 8 >= m->n_expert && (long)m->n_expert * moe_wide_groups(m) >= 512 &&
+           q6k_wide_fits(m->n_ff, m->be) && q6k_wide_fits(m->n_embd, m->bf);
 }
 
 // The expert-grouped FFN of n_tok tokens with routing ids / weights
@@ -1092,22 +1101,26 @@ int moe_grouped(MoeLayer *m, const float *d_x, const int32_t *d_ids, const float
     }
     hipStream_t st = stream();
     const int max_chunks = np / CHUNK + m->n_expert;
-    // up to 4 pairs per expert, most groups are a token or two
     // Exact GEMMs by chunks, with kernels for groups of one and two tokens, up
     // to 12 pairs per expert; twins beyond. Measured per call (us, twins ->
     // few; 128 experts, top 8): 16 tokens 121.6 -> 113.8, 45 117.8 -> 106.0,
     // 80 150.9 -> 138.4, 150 164.3 -> 154.7, 200 171 -> 165, 256 177..196 ->
     // 184..197, 512 256 -> 292.
     const bool few = np <= 12 * m->n_expert;
+    // wide units on few experts: as many as find a CU each, so that a prompt
+    // whose tokens all take the same experts has its chunks side by side (8
+    // experts of 128 for 128 tokens: 60 -> 49 us, twins 55; 4 of 32: 68 -> 51,
+    // twins 51)
+    const bool wide = fast && moe_wide(m, np);
     int rc = 0;
     rc |= launch_moe_group(d_ids, np, m->n_used, m->n_expert, m->p_grp_e.as<int32_t>(),
                            m->p_grp_s.as<int32_t>(), m->p_grp_c.as<int32_t>(),
                            m->p_sub.as<int32_t>(), m->p_slot.as<int32_t>(), m->p_idx.as<int32_t>(),
-                           st, max_chunks);
+                           st, max_chunks, wide ? 256 / moe_wide_groups(m) : 0);
     // Q8_K of every token, written to the chunk slot of each of its n_used pairs
     rc |= launch_q8k_quantize_chunks(d_x, n_tok, m->be, m->p_slot.as<int32_t>(), m->n_used,
                                      m->p_xq.as<int8_t>(), m->p_xd.as<float>(), st);
-    if (fast && moe_wide(m, np)) {
+    if (wide) {
         // gate, up and SwiGLU in one launch, Q8_K of its rows, down
         rc |= launch_q6k_mv_batched_wide(m->gate, m->upw, m->sgu, m->p_sub.as<int32_t>(),
                                          m->p_idx.as<int32_t>(), m->p_xq.as<int8_t>(), m->p_xd.as<float>(),

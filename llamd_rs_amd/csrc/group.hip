@@ -20,8 +20,8 @@
 //   e), pair_idx[i] = the pair index t * n_used + k at sorted position i.
 // With max_chunks > 0, sub_start continues with a record per chunk,
 // sub_info[max_chunks], then one per twin, twin_info[max_chunks], then one per
-// wide unit (up to GROUP_WIDE_CHUNKS chunks, an expert's chunks split evenly)
-// (GroupItem, launch.hpp): a wave of the batched kernels reads its work item in one load
+// wide unit (up to GROUP_WIDE_CHUNKS chunks, fewer where units are few; an
+// expert's chunks split evenly) (GroupItem, launch.hpp): a wave of the batched kernels reads its work item in one load
 // instead of a binary search of dependent loads and the group's fields.
 #include "common.hpp"
 #include "launch.hpp"
@@ -35,7 +35,8 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
                                                   int n_expert, int32_t *grp_expert,
                                                   int32_t *grp_start, int32_t *grp_count,
                                                   int32_t *sub_start, int32_t *slot_of_pair,
-                                                  int32_t *pair_idx, int max_chunks, int max_sorted) {
+                                                  int32_t *pair_idx, int max_chunks, int wide_few,
+                                                  int max_sorted) {
     __shared__ int sub_lds[GROUP_MAX_EXPERTS];
     __shared__ int start_lds[GROUP_MAX_EXPERTS];
     (void)n_used;
@@ -72,16 +73,18 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
     // exclusive prefix sums over experts (thread e owns expert e) of the
     // pair counts and of the 16-token chunk counts
     __shared__ int wsum_c[GROUP_MAX_EXPERTS / WAVE], wsum_s[GROUP_MAX_EXPERTS / WAVE],
-        wsum_t[GROUP_MAX_EXPERTS / WAVE], wsum_u[GROUP_MAX_EXPERTS / WAVE];
+        wsum_t[GROUP_MAX_EXPERTS / WAVE], wsum_q[GROUP_MAX_EXPERTS / WAVE], wsum_u[GROUP_MAX_EXPERTS / WAVE];
     const int lane = tid & 63, wave = tid >> 6;
     const int c = tid < n_expert ? hist[tid] : 0, ch = (c + 15) / 16, tw = (ch + 1) / 2;
-    const int wu = (ch + GROUP_WIDE_CHUNKS - 1) / GROUP_WIDE_CHUNKS;
+    const int qu = (ch + 3) / 4;
+    int wu = (ch + GROUP_WIDE_CHUNKS - 1) / GROUP_WIDE_CHUNKS;
     const int ic = wave_incl_sum_i(c), is = wave_incl_sum_i(ch), it = wave_incl_sum_i(tw);
-    const int iu = wave_incl_sum_i(wu);
+    const int iu = wave_incl_sum_i(wu), iq = wide_few > 0 ? wave_incl_sum_i(qu) : 0;
     if (lane == WAVE - 1) {
         wsum_c[wave] = ic;
         wsum_s[wave] = is;
         wsum_t[wave] = it;
+        wsum_q[wave] = iq;
         wsum_u[wave] = iu;
     }
     __syncthreads();
@@ -91,6 +94,26 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
         sub += wsum_s[w];
         tst += wsum_t[w];
         ust += wsum_u[w];
+    }
+    if (wide_few > 0) {
+        // shorter wide units where those of 1, 2 or 4 chunks are few as well
+        int s1 = 0, s2 = 0, s4 = 0, before = 0;
+        for (int w = 0; WAVE * w < n_expert; ++w) {
+            s1 += wsum_s[w];
+            s2 += wsum_t[w];
+            s4 += wsum_q[w];
+            if (w < wave) before += wsum_q[w];
+        }
+        if (s1 <= wide_few) {
+            wu = ch;
+            ust = sub;
+        } else if (s2 <= wide_few) {
+            wu = tw;
+            ust = tst;
+        } else if (s4 <= wide_few) {
+            wu = qu;
+            ust = before + iq - qu;
+        }
     }
     if (tid < n_expert) {
         grp_expert[tid] = tid;
@@ -175,7 +198,8 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
 int launch_moe_group(const int32_t *ids, int n_pairs, int n_used, int n_expert,
                      int32_t *grp_expert, int32_t *grp_start, int32_t *grp_count,
                      int32_t *sub_start, int32_t *slot_of_pair, int32_t *pair_idx,
-                     hipStream_t st, int max_chunks) {
+                     hipStream_t st, int max_chunks, int wide_few) {
+    if (wide_few > n_expert) return -1;  // (group_wide_units)
     if (n_expert > GROUP_MAX_EXPERTS || n_expert <= 0 || max_chunks < 0) return -1;
     const int max_sorted = 24576;
     const size_t lds = n_pairs > 8192 && n_pairs <= max_sorted ? (size_t)n_pairs * 4 : 0;
@@ -184,7 +208,7 @@ int launch_moe_group(const int32_t *ids, int n_pairs, int n_used, int n_expert,
     if (ok != hipSuccess) return -1;
     hipLaunchKernelGGL(moe_group, dim3(1), dim3(1024), lds, st, ids, n_pairs, n_used, n_expert,
                        grp_expert, grp_start, grp_count, sub_start, slot_of_pair, pair_idx,
-                       max_chunks, max_sorted);
+                       max_chunks, wide_few, max_sorted);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -130,6 +130,8 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
 // w2 set: y = silu(w . a) * (w2 . a) instead. y [pairs][rows], 16-byte aligned.
 constexpr int WIDE_MAX_BLOCKS = 16;
 bool q6k_wide_fits(int rows, int blocks);
+// Workgroups that a unit makes of these rows.
+int q6k_wide_groups(int rows, bool pair);
 int launch_q6k_mv_batched_wide(const void *w, const void *w2, size_t expert_stride,
                                const int32_t *sub_start, const int32_t *pair_out,
                                const int8_t *act_q, const float *act_d, float *y, int rows,
@@ -195,6 +197,8 @@ struct __attribute__((aligned(32))) GroupItem {
 constexpr size_t group_items_offset(int n_expert) { return ((2 * (size_t)(n_expert + 1)) + 7) & ~(size_t)7; }
 // Wide units: up to this many consecutive chunks of one expert, and the
 // records (a multiple of 8) that any grouping into max_chunks chunks takes.
+// Where the routing leaves few units, they are shorter: 1, 2 or 4 chunks at
+// most, the least that makes no more than wide_few units (at most n_expert).
 constexpr int GROUP_WIDE_CHUNKS = 8;
 constexpr int group_wide_units(int n_expert, int max_chunks) {
     return (max_chunks / GROUP_WIDE_CHUNKS + n_expert + 7) / 8 * 8;
@@ -207,7 +211,7 @@ constexpr size_t group_table_size(int n_expert, int max_chunks) {
 int launch_moe_group(const int32_t *ids, int n_pairs, int n_used, int n_expert,
                      int32_t *grp_expert, int32_t *grp_start, int32_t *grp_count,
                      int32_t *sub_start, int32_t *slot_of_pair, int32_t *pair_idx,
-                     hipStream_t st, int max_chunks = 0);
+                     hipStream_t st, int max_chunks = 0, int wide_few = 0);
 int launch_silu_mul(const float *gate, const float *up, float *out, int n, hipStream_t st);
 
 // norm.hip: CpuBackend::rms_norm (+ weight), bit-exact. rows of n; the

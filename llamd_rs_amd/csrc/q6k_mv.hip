@@ -2239,6 +2239,11 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+int q6k_wide_groups(int rows, bool pair) {
+    const int tiles = (rows + TILE_ROWS - 1) / TILE_ROWS;
+    return pair ? (tiles + 3) / 4 : (tiles + 7) / 8;  // four of gate and four of up, or eight
+}
+
 bool q6k_wide_fits(int rows, int blocks) { return rows % TILE_ROWS == 0 && blocks <= WIDE_MAX_BLOCKS; }
 
 int launch_q6k_mv_batched_wide(const void *w, const void *w2, size_t expert_stride,
@@ -2258,7 +2263,7 @@ int launch_q6k_mv_batched_wide(const void *w, const void *w2, size_t expert_stri
     p.ldy = p.rows = rows;
     p.tiles = rows / TILE_ROWS;
     p.blocks = blocks;
-    const int row_groups = w2 ? (p.tiles + 3) / 4 : (p.tiles + 7) / 8;
+    const int row_groups = q6k_wide_groups(rows, w2 != nullptr);
     const int units = group_wide_units(n_groups, max_chunks);
     constexpr size_t lds = 2 * WIDE_CHUNKS * CHUNK_BLOCK_BYTES;
     if (w2) hipLaunchKernelGGL(q6k_mv_batched_wide<true>, dim3(units * row_groups), dim3(512), lds, st, p, row_groups);

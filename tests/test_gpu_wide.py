@@ -52,6 +52,27 @@ def test_grouped_edges_of_chunks_twins_and_units(gpu):
     assert np.linalg.norm(red - got) / np.linalg.norm(got) < 1e-3
 
 
+@pytest.mark.parametrize("n_tok,n_used,taken", [(256, 4, 4), (129, 8, 8), (330, 8, 8), (700, 8, 12), (150, 8, 100)])
+def test_reduction_wide_units_of_few_experts(gpu, n_tok, n_used, taken):
+    """`taken` of 128 experts take the prompt, so that wide units have up to 1,
+    2, 4, 8 and 8 chunks: rows within the REDUCTION tolerance of the bit-exact
+    ones, and the same bits with the tokens in another order."""
+    n_embd, n_ff, n_expert = 512, 256, 128
+    m, _ = layer(gpu, n_embd, n_ff, n_expert, n_used, 970)
+    rng = np.random.default_rng(n_tok)
+    names = rng.permutation(n_expert)[:taken]
+    ids = np.stack([rng.permutation(names)[:n_used] for _ in range(n_tok)]).astype(np.int32)
+    x = (H.sample(n_tok * n_embd, 16) * 2).astype(np.float32).reshape(n_tok, n_embd)
+    w = (H.sample(n_tok * n_used, 17).reshape(n_tok, n_used) + np.float32(2)).astype(np.float32)
+    L = gpu.lib()
+    got = prefill(L, gpu, m, x, ids, w, 0)
+    red = prefill(L, gpu, m, x, ids, w, 1)
+    assert np.linalg.norm(red - got) / np.linalg.norm(got) < 1e-3
+    turn = rng.permutation(n_tok)
+    again = prefill(L, gpu, m, x[turn].copy(), ids[turn].copy(), w[turn].copy(), 1)
+    assert np.array_equal(again.view(np.uint32), red[turn].view(np.uint32))
+
+
 @pytest.mark.parametrize("n_tok,n_used", [(1024, 8), (1025, 8), (3073, 8), (64, 2)])
 def test_grouped_prompt_lengths(gpu, n_tok, n_used):
     """Past 8192 and 24576 pairs the sort takes its other routes: every token's
