@@ -1111,7 +1111,8 @@ int moe_grouped(MoeLayer *m, const float *d_x, const int32_t *d_ids, const float
     // whose tokens all take the same experts has its chunks side by side (8
     // experts of 128 for 128 tokens: 60 -> 49 us, twins 55; 4 of 32: 68 -> 51,
     // twins 51)
-    const bool wide = fast && moe_wide(m, np);
+    // (batched_twin 0: one chunk per wave in every grouped GEMM)
+    const bool wide = fast && g_tune_batched_twin && moe_wide(m, np);
     int rc = 0;
     rc |= launch_moe_group(d_ids, np, m->n_used, m->n_expert, m->p_grp_e.as<int32_t>(),
                            m->p_grp_s.as<int32_t>(), m->p_grp_c.as<int32_t>(),

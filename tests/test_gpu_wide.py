@@ -27,11 +27,26 @@ def prefill(L, gpu, m, x, ids, w, flags):
     return out.download(np.empty_like(x))
 
 
-def test_grouped_edges_of_chunks_twins_and_units(gpu):
+def by_chunks(L, gpu, m, x, ids, w, flags):
+    """The same call with a 16-token chunk per wave."""
+    prev = L.llamd_hip_tune(b"batched_twin", 0)
+    try:
+        return prefill(L, gpu, m, x, ids, w, flags)
+    finally:
+        L.llamd_hip_tune(b"batched_twin", prev)
+
+
+EDGES = [0, 1, 2, 3, 15, 16, 17, 32, 33, 128, 129, 145]
+
+
+@pytest.mark.parametrize("n_embd,n_ff,counts", [
+    (768, 256, EDGES),                                         # twins
+    (512, 256, EDGES + [255, 256, 257] + [0] * 113),           # REDUCTION: wide units of 2 chunks
+    (512, 256, EDGES + [255, 256, 257] + [18] * 60 + [0] * 53)])  # of 8
+def test_grouped_edges_of_chunks_twins_and_units(gpu, n_embd, n_ff, counts):
     """Exact rows equal the CPU's; REDUCTION rows differ from them by the f32
     rounding of nb terms and by quants of the SwiGLU output that it moves: one
     step of 1/127 of a block's largest value, on one of its 256 values."""
-    n_embd, n_ff, counts = 768, 256, [0, 1, 2, 3, 15, 16, 17, 32, 33, 128, 129, 145]
     n_expert = len(counts)
     m, (gate, up, down) = layer(gpu, n_embd, n_ff, n_expert, 1, 900)
     ids = np.repeat(np.arange(n_expert, dtype=np.int32), counts)[:, None]
@@ -50,6 +65,30 @@ def test_grouped_edges_of_chunks_twins_and_units(gpu):
     rms = np.sqrt((got[:-2].astype(np.float64) ** 2).mean(1, keepdims=True))
     assert (np.abs(red[:-2] - got[:-2]) / rms).max() < 3e-2
     assert np.linalg.norm(red - got) / np.linalg.norm(got) < 1e-3
+    assert np.array_equal(by_chunks(L, gpu, m, x, ids, w, 0).view(np.uint32), got.view(np.uint32))
+    assert np.array_equal(by_chunks(L, gpu, m, x, ids, w, 1).view(np.uint32), red.view(np.uint32))
+
+
+@pytest.mark.parametrize("counts", [(17, 1, 64, 2, 33, 3), (32, 31, 16, 49)])
+def test_grouped_edges_of_mostly_empty_experts(gpu, counts):
+    """Fewer than 8 pairs per expert, so exact rows take the kernel for groups of
+    one and two tokens and REDUCTION rows the twins, with some experts of more
+    than a chunk: exact rows equal the CPU's, REDUCTION rows are the same bits by
+    twins and by chunks."""
+    n_embd, n_ff, n_expert = 512, 256, 64
+    m, (gate, up, down) = layer(gpu, n_embd, n_ff, n_expert, 1, 930)
+    ids = np.repeat(3 * np.arange(len(counts), dtype=np.int32) + 1, counts)[:, None]
+    ids = ids[np.argsort(H.sample(len(ids), 18))].copy()
+    n = len(ids)
+    x = (H.sample(n * n_embd, 19) * 2).astype(np.float32).reshape(n, n_embd)
+    w = (H.sample(n, 20).reshape(n, 1) + np.float32(2)).astype(np.float32)
+    L = gpu.lib()
+    got = prefill(L, gpu, m, x, ids, w, 0)
+    want = O.moe_ffn_tokens(x, n_embd, n_ff, n_expert, gate, up, down, ids.astype(np.uint32), w)
+    assert np.array_equal(got.view(np.uint32), np.asarray(want, np.float32).reshape(-1, n_embd).view(np.uint32))
+    red = prefill(L, gpu, m, x, ids, w, 1)
+    assert np.linalg.norm(red - got) / np.linalg.norm(got) < 1e-3
+    assert np.array_equal(by_chunks(L, gpu, m, x, ids, w, 1).view(np.uint32), red.view(np.uint32))
 
 
 @pytest.mark.parametrize("n_tok,n_used,taken", [(256, 4, 4), (129, 8, 8), (330, 8, 8), (700, 8, 12), (150, 8, 100)])
@@ -68,6 +107,7 @@ def test_reduction_wide_units_of_few_experts(gpu, n_tok, n_used, taken):
     got = prefill(L, gpu, m, x, ids, w, 0)
     red = prefill(L, gpu, m, x, ids, w, 1)
     assert np.linalg.norm(red - got) / np.linalg.norm(got) < 1e-3
+    assert np.array_equal(by_chunks(L, gpu, m, x, ids, w, 1).view(np.uint32), red.view(np.uint32))
     turn = rng.permutation(n_tok)
     again = prefill(L, gpu, m, x[turn].copy(), ids[turn].copy(), w[turn].copy(), 1)
     assert np.array_equal(again.view(np.uint32), red[turn].view(np.uint32))
@@ -76,9 +116,10 @@ def test_reduction_wide_units_of_few_experts(gpu, n_tok, n_used, taken):
 @pytest.mark.parametrize("n_tok,n_used", [(1024, 8), (1025, 8), (3073, 8), (64, 2)])
 def test_grouped_prompt_lengths(gpu, n_tok, n_used):
     """Past 8192 and 24576 pairs the sort takes its other routes: every token's
-    row equals the row it gets in a call of 64 tokens."""
+    row equals the row it gets in a call of 64 tokens, and those of the last 64
+    are the CPU's."""
     n_embd, n_ff, n_expert = 256, 256, 16
-    m, _ = layer(gpu, n_embd, n_ff, n_expert, n_used, 950)
+    m, (gate, up, down) = layer(gpu, n_embd, n_ff, n_expert, n_used, 950)
     x = (H.sample(n_tok * n_embd, 8) * 2).astype(np.float32).reshape(n_tok, n_embd)
     score = H.sample(n_tok * n_expert, 9).reshape(n_tok, n_expert)
     ids = np.argsort(-score, axis=1)[:, :n_used].astype(np.int32)
@@ -89,6 +130,8 @@ def test_grouped_prompt_lengths(gpu, n_tok, n_used):
         s = slice(a, a + 64)
         part = prefill(L, gpu, m, x[s].copy(), ids[s].copy(), w[s].copy(), 0)
         assert np.array_equal(part.view(np.uint32), whole[s].view(np.uint32)), a
+    want = O.moe_ffn_tokens(x[s], n_embd, n_ff, n_expert, gate, up, down, ids[s].astype(np.uint32), w[s])
+    assert np.array_equal(part.view(np.uint32), np.asarray(want, np.float32).reshape(-1, n_embd).view(np.uint32))
     red = prefill(L, gpu, m, x, ids, w, 1)
     assert np.linalg.norm(red - whole) / np.linalg.norm(whole) < 1e-3
 
