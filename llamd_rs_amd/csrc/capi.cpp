@@ -165,7 +165,7 @@ size_t chunk_d_bytes(int nseq, int blocks) {
 // Single-group batched matvec: all rows, nseq tokens in chunk slots 0..nseq-1.
 int batched_dev(const void *w, const int8_t *cq, const float *cd, float *y, int blocks, int rows,
                 int nseq) {
-    return launch_q6k_mv_batched(w, 0, nullptr, nullptr, nullptr, nullptr, nullptr, cq, cd, y, rows,
+    return launch_q6k_mv_batched(w, 0, nullptr, nullptr, cq, cd, y, rows,
                                  rows, blocks, nseq, (nseq + CHUNK - 1) / CHUNK, stream());
 }
 
@@ -825,7 +825,7 @@ struct MoeLayer {
     bool decode_fits() const { return bf <= 8 && be <= 8; }
     // prefill scratch (grown on demand)
     int cap_tok = 0, cap_seq = 1;  // prefill tokens; decode sequences (logits .. slots below)
-    DevBuf p_xq, p_xd, p_grp_e, p_grp_s, p_grp_c, p_sub, p_slot, p_idx, p_g, p_u, p_aq, p_ad, p_dn;
+    DevBuf p_xq, p_xd, p_rec, p_slot, p_idx, p_g, p_u, p_aq, p_ad, p_dn;
 };
 
 // The decode kernels' arguments for this layer's scratch.
@@ -1089,8 +1089,7 @@ int moe_grouped(MoeLayer *m, const float *d_x, const int32_t *d_ids, const float
         const int chunks = np / CHUNK + m->n_expert;  // bound on sum of ceil(count/16)
         bool ok = m->p_xq.alloc((size_t)chunks * m->be * CHUNK_BLOCK) &&
                   m->p_xd.alloc((size_t)chunks * m->be * CHUNK * 4) &&
-                  m->p_grp_e.alloc(m->n_expert * 4) && m->p_grp_s.alloc(m->n_expert * 4) &&
-                  m->p_grp_c.alloc(m->n_expert * 4) && m->p_sub.alloc(group_table_size(m->n_expert, chunks) * 4) &&
+                  m->p_rec.alloc(group_records(m->n_expert, chunks) * sizeof(GroupItem)) &&
                   m->p_slot.alloc(NP * 4) && m->p_idx.alloc(NP * 4) &&
                   m->p_g.alloc(NP * m->n_ff * 4) && m->p_u.alloc(NP * m->n_ff * 4) &&
                   m->p_aq.alloc((size_t)chunks * m->bf * CHUNK_BLOCK) &&
@@ -1114,44 +1113,39 @@ int moe_grouped(MoeLayer *m, const float *d_x, const int32_t *d_ids, const float
     // (batched_twin 0: one chunk per wave in every grouped GEMM)
     const bool wide = fast && g_tune_batched_twin && moe_wide(m, np);
     int rc = 0;
-    rc |= launch_moe_group(d_ids, np, m->n_used, m->n_expert, m->p_grp_e.as<int32_t>(),
-                           m->p_grp_s.as<int32_t>(), m->p_grp_c.as<int32_t>(),
-                           m->p_sub.as<int32_t>(), m->p_slot.as<int32_t>(), m->p_idx.as<int32_t>(),
-                           st, max_chunks, wide ? 256 / moe_wide_groups(m) : 0);
+    rc |= launch_moe_group(d_ids, np, m->n_expert, m->p_rec.as<GroupItem>(), m->p_slot.as<int32_t>(),
+                           m->p_idx.as<int32_t>(), st, max_chunks, wide ? 256 / moe_wide_groups(m) : 0);
     // Q8_K of every token, written to the chunk slot of each of its n_used pairs
     rc |= launch_q8k_quantize_chunks(d_x, n_tok, m->be, m->p_slot.as<int32_t>(), m->n_used,
                                      m->p_xq.as<int8_t>(), m->p_xd.as<float>(), st);
     if (wide) {
         // gate, up and SwiGLU in one launch, Q8_K of its rows, down
-        rc |= launch_q6k_mv_batched_wide(m->gate, m->upw, m->sgu, m->p_sub.as<int32_t>(),
+        rc |= launch_q6k_mv_batched_wide(m->gate, m->upw, m->sgu, m->p_rec.as<GroupItem>(),
                                          m->p_idx.as<int32_t>(), m->p_xq.as<int8_t>(), m->p_xd.as<float>(),
                                          m->p_g.as<float>(), m->n_ff, m->be, m->n_expert, max_chunks, st);
         rc |= launch_q8k_quantize_chunks(m->p_g.as<float>(), np, m->bf, m->p_slot.as<int32_t>(), 1,
                                          m->p_aq.as<int8_t>(), m->p_ad.as<float>(), st);
-        rc |= launch_q6k_mv_batched_wide(m->downw, nullptr, m->sd, m->p_sub.as<int32_t>(),
+        rc |= launch_q6k_mv_batched_wide(m->downw, nullptr, m->sd, m->p_rec.as<GroupItem>(),
                                          m->p_idx.as<int32_t>(), m->p_aq.as<int8_t>(), m->p_ad.as<float>(),
                                          m->p_dn.as<float>(), m->n_embd, m->bf, m->n_expert, max_chunks, st);
         rc |= launch_moe_combine(m->p_dn.as<float>(), d_w, d_res, d_out, m->n_used, m->n_embd, n_tok, st,
                                  m->p_slot.as<int32_t>());
         return rc ? fail("moe_prefill: launch failed") : 0;
     }
-    // gate / up: output row = the pair index
-    // gate and up in one launch (same shapes, same activations)
-    rc |= launch_q6k_mv_batched(m->gate, m->sgu, m->p_grp_e.as<int32_t>(), m->p_grp_s.as<int32_t>(),
-                                m->p_grp_c.as<int32_t>(), m->p_sub.as<int32_t>(),
-                                m->p_idx.as<int32_t>(), m->p_xq.as<int8_t>(), m->p_xd.as<float>(),
-                                m->p_g.as<float>(), m->n_ff, m->n_ff, m->be, m->n_expert, max_chunks, st,
-                                nullptr, nullptr, true, m->upw, m->p_u.as<float>(), fast, few);
+    // gate and up in one launch (same shapes, same activations); output row = the
+    // pair index
+    rc |= launch_q6k_mv_batched(m->gate, m->sgu, m->p_rec.as<GroupItem>(), m->p_idx.as<int32_t>(),
+                                m->p_xq.as<int8_t>(), m->p_xd.as<float>(), m->p_g.as<float>(), m->n_ff,
+                                m->n_ff, m->be, m->n_expert, max_chunks, st, nullptr, nullptr, m->upw,
+                                m->p_u.as<float>(), fast, few);
     // SwiGLU + Q8_K per pair, into the pair's chunk slot
     rc |= launch_swiglu_q8k_chunks(m->p_g.as<float>(), m->p_u.as<float>(), np, m->bf,
                                    m->p_slot.as<int32_t>(), m->p_aq.as<int8_t>(),
                                    m->p_ad.as<float>(), st);
-    // down: output row = the pair index
-    rc |= launch_q6k_mv_batched(m->downw, m->sd, m->p_grp_e.as<int32_t>(), m->p_grp_s.as<int32_t>(),
-                                m->p_grp_c.as<int32_t>(), m->p_sub.as<int32_t>(),
-                                m->p_idx.as<int32_t>(), m->p_aq.as<int8_t>(), m->p_ad.as<float>(),
-                                m->p_dn.as<float>(), m->n_embd, m->n_embd, m->bf, m->n_expert,
-                                max_chunks, st, nullptr, nullptr, true, nullptr, nullptr, fast, few);
+    rc |= launch_q6k_mv_batched(m->downw, m->sd, m->p_rec.as<GroupItem>(), m->p_idx.as<int32_t>(),
+                                m->p_aq.as<int8_t>(), m->p_ad.as<float>(), m->p_dn.as<float>(), m->n_embd,
+                                m->n_embd, m->bf, m->n_expert, max_chunks, st, nullptr, nullptr, nullptr,
+                                nullptr, fast, few);
     rc |= launch_moe_combine(m->p_dn.as<float>(), d_w, d_res, d_out, m->n_used, m->n_embd, n_tok, st,
                              m->p_slot.as<int32_t>());
     return rc ? fail("moe_prefill: launch failed") : 0;
@@ -1276,15 +1270,15 @@ int llamd::lmhead_enqueue(const void *w, int rows, int blocks, const float *d_x,
     } else if (sc.mt) {
         // REDUCTION-tolerance logits; the arg-max is certified and exact
         rc |= launch_q8k_quantize_chunks(d_x, nseq, blocks, nullptr, 1, sc.cq, sc.cd, st, sc.xq, sc.xd);
-        rc |= launch_q6k_mv_batched(w, 0, nullptr, nullptr, nullptr, nullptr, nullptr, sc.cq, sc.cd,
+        rc |= launch_q6k_mv_batched(w, 0, nullptr, nullptr, sc.cq, sc.cd,
                                     d_logits, rows, rows, blocks, nseq, (nseq + CHUNK - 1) / CHUNK,
-                                    st, sc.pv, sc.pi, false, nullptr, nullptr, true);
+                                    st, sc.pv, sc.pi, nullptr, nullptr, true);
         rc |= launch_lmhead_certify(w, rows, blocks, nseq, sc.xq, sc.xd, sc.pv, sc.pi, sc.mt,
                                     d_logits, d_ids, st);
         return rc;
     } else {
         rc |= launch_q8k_quantize_chunks(d_x, nseq, blocks, nullptr, 1, sc.cq, sc.cd, st);
-        rc |= launch_q6k_mv_batched(w, 0, nullptr, nullptr, nullptr, nullptr, nullptr, sc.cq, sc.cd,
+        rc |= launch_q6k_mv_batched(w, 0, nullptr, nullptr, sc.cq, sc.cd,
                                     d_logits, rows, rows, blocks, nseq, (nseq + CHUNK - 1) / CHUNK,
                                     st, sc.pv, sc.pi);
     }

@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256) void act_unbias(const uint32_t *q, uint32_t fl
 }
 
 // Natural-layout quants and scales of n_act tokens -> the token-chunked
-// operand layout of q6k_mv_batched (chunk_byte, q8k_wave.hpp). Token slots past
+// operand layout of the batched matvecs (chunk_byte, q8k_wave.hpp). Token slots past
 // n_act are zero.
 __global__ __launch_bounds__(256) void act_to_chunks(const uint8_t *q, const float *d, uint8_t flip,
                                                      int n_act, int blocks, uint8_t *cq, float *cd,

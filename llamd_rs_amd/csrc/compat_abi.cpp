@@ -225,7 +225,7 @@ int chunked(const void *q, const float *d, bool biased, int n_act, int blocks, A
 int matvec_n(const Q6kView &v, const Acts &a, float *out, int rows, int blocks, int nseq) {
     if (nseq == 1)
         return launch_q6k_mv_b1(v.tiled, 0, nullptr, a.q, a.d, out, rows, blocks, 1, 0, S());
-    return launch_q6k_mv_batched(v.tiled, 0, nullptr, nullptr, nullptr, nullptr, nullptr, a.cq, a.cd,
+    return launch_q6k_mv_batched(v.tiled, 0, nullptr, nullptr, a.cq, a.cd,
                                  out, rows, rows, blocks, nseq, (nseq + CHUNK - 1) / CHUNK, S());
 }
 

@@ -10,19 +10,14 @@
 // exactly, the property crates/llamd-testing/tests/vulkan_prefill.rs:268-333
 // holds the reference's Vulkan path to.
 //
-// Outputs (all experts are groups, empty ones included):
-//   grp_expert[e] = e, grp_start[e], grp_count[e],
-//   sub_start[0..n_expert] = prefix sum of ceil(count/16) (16-token chunks
-//   of the batched kernel), followed by twin_start = sub_start[n_expert + 1
-//   .. 2 n_expert + 1] = prefix sum of ceil(chunks/2) (twins: two chunks of
-//   one expert, the work items of the twin batched kernel), slot_of_pair[p] = the chunk slot of pair p
-//   (chunk sub_start[e] + j / 16, token j % 16 for the j-th pair of expert
-//   e), pair_idx[i] = the pair index t * n_used + k at sorted position i.
-// With max_chunks > 0, sub_start continues with a record per chunk,
-// sub_info[max_chunks], then one per twin, twin_info[max_chunks], then one per
-// wide unit (up to GROUP_WIDE_CHUNKS chunks, fewer where units are few; an
-// expert's chunks split evenly) (GroupItem, launch.hpp): a wave of the batched kernels reads its work item in one load
-// instead of a binary search of dependent loads and the group's fields.
+// Outputs: slot_of_pair[p] = the chunk slot of pair p (an expert's 16-token chunks
+// follow the expert before's; the j-th pair of an expert is token j % 16 of its
+// chunk j / 16), pair_idx[i] = the pair index t * n_used + k at sorted position i,
+// and a record per work item of the batched kernels (GroupItem, launch.hpp), which
+// a wave reads in one load: one per chunk, records[max_chunks], then one per twin
+// (two chunks of one expert), [max_chunks], then one per wide unit (up to
+// GROUP_WIDE_CHUNKS chunks, fewer where units are few; an expert's chunks split
+// evenly), [group_wide_units].
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -31,15 +26,12 @@ namespace {
 
 constexpr int GROUP_MAX_EXPERTS = 1024;
 
-__global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pairs, int n_used,
-                                                  int n_expert, int32_t *grp_expert,
-                                                  int32_t *grp_start, int32_t *grp_count,
-                                                  int32_t *sub_start, int32_t *slot_of_pair,
+__global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pairs, int n_expert,
+                                                  GroupItem *records, int32_t *slot_of_pair,
                                                   int32_t *pair_idx, int max_chunks, int wide_few,
                                                   int max_sorted) {
     __shared__ int sub_lds[GROUP_MAX_EXPERTS];
     __shared__ int start_lds[GROUP_MAX_EXPERTS];
-    (void)n_used;
     __shared__ int hist[GROUP_MAX_EXPERTS];
     __shared__ int cursor[GROUP_MAX_EXPERTS];
     constexpr int PB = 8;
@@ -115,52 +107,36 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
             ust = before + iq - qu;
         }
     }
+    GroupItem *twin_info = records + max_chunks, *wide_info = twin_info + max_chunks;
     if (tid < n_expert) {
-        grp_expert[tid] = tid;
-        grp_start[tid] = start;
-        grp_count[tid] = c;
-        sub_start[tid] = sub;
-        sub_start[n_expert + 1 + tid] = tst;
         sub_lds[tid] = sub;
         start_lds[tid] = start;
         cursor[tid] = 0;
         if (tid == n_expert - 1) {
-            sub_start[n_expert] = sub + ch;
-            sub_start[2 * n_expert + 1] = tst + tw;
             totals[0] = sub + ch;
             totals[1] = tst + tw;
             totals[2] = start + c;
             totals[3] = ust + wu;
         }
-        if (max_chunks > 0) {
-            GroupItem *sub_info = (GroupItem *)(sub_start + group_items_offset(n_expert));
-            GroupItem *twin_info = sub_info + max_chunks;
-            for (int j = 0; j < ch; ++j)
-                sub_info[sub + j] = GroupItem{tid, j, sub + j, c, start, 0, 0, 0};
-            for (int j = 0; j < tw; ++j)
-                twin_info[tst + j] = GroupItem{tid, 2 * j, sub + 2 * j, c, start, 2 * j + 1 < ch, 0, 0};
-            GroupItem *wide_info = twin_info + max_chunks;
-            for (int j = 0, at = 0; j < wu; ++j) {
-                const int nc = ch / wu + (j < ch % wu);
-                wide_info[ust + j] = GroupItem{tid, at, sub + at, c, start, nc, 0, 0};
-                at += nc;
-            }
+        for (int j = 0; j < ch; ++j)
+            records[sub + j] = GroupItem{tid, j, sub + j, c, start, 0, 0, 0};
+        for (int j = 0; j < tw; ++j)
+            twin_info[tst + j] = GroupItem{tid, 2 * j, sub + 2 * j, c, start, 2 * j + 1 < ch, 0, 0};
+        for (int j = 0, at = 0; j < wu; ++j) {
+            const int nc = ch / wu + (j < ch % wu);
+            wide_info[ust + j] = GroupItem{tid, at, sub + at, c, start, nc, 0, 0};
+            at += nc;
         }
     }
     __syncthreads();
-    if (max_chunks > 0) {
-        // the records past the last chunk / twin: no work (expert -1), so a
-        // wave of the grid's spare items needs no other load to know it
-        GroupItem *sub_info = (GroupItem *)(sub_start + group_items_offset(n_expert));
-        GroupItem *twin_info = sub_info + max_chunks;
-        for (int i = totals[0] + tid; i < max_chunks; i += blockDim.x)
-            sub_info[i] = GroupItem{-1, 0, 0, 0, 0, 0, 0, 0};
-        for (int i = totals[1] + tid; i < max_chunks; i += blockDim.x)
-            twin_info[i] = GroupItem{-1, 0, 0, 0, 0, 0, 0, 0};
-        GroupItem *wide_info = twin_info + max_chunks;
-        for (int i = totals[3] + tid; i < group_wide_units(n_expert, max_chunks); i += blockDim.x)
-            wide_info[i] = GroupItem{-1, 0, 0, 0, 0, 0, 0, 0};
-    }
+    // the records past the last chunk / twin / unit: no work (expert -1), so a
+    // wave of the grid's spare items needs no other load to know it
+    for (int i = totals[0] + tid; i < max_chunks; i += blockDim.x)
+        records[i] = GroupItem{-1, 0, 0, 0, 0, 0, 0, 0};
+    for (int i = totals[1] + tid; i < max_chunks; i += blockDim.x)
+        twin_info[i] = GroupItem{-1, 0, 0, 0, 0, 0, 0, 0};
+    for (int i = totals[3] + tid; i < group_wide_units(n_expert, max_chunks); i += blockDim.x)
+        wide_info[i] = GroupItem{-1, 0, 0, 0, 0, 0, 0, 0};
     for (int base = 0; base < n_pairs; base += PB * (int)blockDim.x) {
         if (!once) {
             // more pairs than registers: the ids and their places again
@@ -195,20 +171,18 @@ __global__ __launch_bounds__(1024) void moe_group(const int32_t *ids, int n_pair
 
 }  // namespace
 
-int launch_moe_group(const int32_t *ids, int n_pairs, int n_used, int n_expert,
-                     int32_t *grp_expert, int32_t *grp_start, int32_t *grp_count,
-                     int32_t *sub_start, int32_t *slot_of_pair, int32_t *pair_idx,
-                     hipStream_t st, int max_chunks, int wide_few) {
+int launch_moe_group(const int32_t *ids, int n_pairs, int n_expert, GroupItem *records,
+                     int32_t *slot_of_pair, int32_t *pair_idx, hipStream_t st, int max_chunks,
+                     int wide_few) {
     if (wide_few > n_expert) return -1;  // (group_wide_units)
-    if (n_expert > GROUP_MAX_EXPERTS || n_expert <= 0 || max_chunks < 0) return -1;
+    if (n_expert > GROUP_MAX_EXPERTS || n_expert <= 0 || max_chunks <= 0) return -1;
     const int max_sorted = 24576;
     const size_t lds = n_pairs > 8192 && n_pairs <= max_sorted ? (size_t)n_pairs * 4 : 0;
     static const hipError_t ok = hipFuncSetAttribute((const void *)moe_group, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                      max_sorted * 4);
     if (ok != hipSuccess) return -1;
-    hipLaunchKernelGGL(moe_group, dim3(1), dim3(1024), lds, st, ids, n_pairs, n_used, n_expert,
-                       grp_expert, grp_start, grp_count, sub_start, slot_of_pair, pair_idx,
-                       max_chunks, wide_few, max_sorted);
+    hipLaunchKernelGGL(moe_group, dim3(1), dim3(1024), lds, st, ids, n_pairs, n_expert, records,
+                       slot_of_pair, pair_idx, max_chunks, wide_few, max_sorted);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -18,9 +18,9 @@ __host__ __device__ constexpr int chunk_byte(int e, int n) {
 }
 
 // Tuning overrides (0 = automatic); set through llamd_hip_tune.
-extern int g_tune_batched_twin;
+extern int g_tune_batched_twin;  // grouped GEMMs: two chunks of one expert per wave
 extern int g_tune_fast_lds;  // LLAMD_HIP_REDUCTION LM head: the chunk's quants staged in LDS
-extern int g_tune_fast_ks;  // LLAMD_HIP_REDUCTION batched kernels: waves per item (K split), 0 = by shape  // grouped q6k_mv_batched: two chunks of one expert per wave
+extern int g_tune_fast_ks;  // LLAMD_HIP_REDUCTION batched kernels: waves per item (K split), 0 = by shape
 extern int g_tune_mv_ks;  // waves per 16-row tile in q6k_mv_b1: 1, 2, 4 or 8 (0: automatic)
 extern int g_tune_model_graph;  // 1: the decode step of llamd_hip_model_* is a captured graph
 extern int g_tune_model_fused_attn;  // 1: attend_fused in the decode step
@@ -61,14 +61,6 @@ int launch_q6k_down_combine(const void *w, size_t expert_stride, const int32_t *
                             const int8_t *aq, const float *ad, const float *weights,
                             const float *res, float *out, int rows, int blocks, int n_slots,
                             hipStream_t st);
-// Expert-grouped batched matvec (see q6k_mv.hip). Activations are in the
-// token-chunked layout (q8k_wave.hpp): chunk k holds the 16 tokens of
-// sub-tile k. sub_start has 2 * (n_groups + 1) entries: the prefix of
-// ceil(count/16) per group, then (read while g_tune_batched_twin is on) the
-// prefix of ceil(chunks/2), as launch_moe_group writes them; max_chunks bounds
-// sub_start[n_groups] and sizes the grid. The output of the
-// pair at sorted position i is row pair_out[i] of y (nullptr: row i). With
-// grp_expert == nullptr there is a single group (expert 0) of n_groups tokens.
 // moe_decode.hip: one MoE decode layer (router, top-k, gate, up, SwiGLU,
 // down, combine, residual) in two launches, bit-identical to the reference.
 struct MoeDecodeLaunch {
@@ -106,24 +98,21 @@ const float *moe_router(void *moe);
 int moe_router_rows(void *moe);
 int moe_forward_normed(void *moe, const float *x, const float *o, const float *w, float eps,
                        float *sum_out, float *out);
-int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *grp_expert,
-                          const int32_t *grp_start, const int32_t *grp_count,
-                          const int32_t *sub_start, const int32_t *pair_out, const int8_t *act_q,
-                          const float *act_d, float *y, int ldy, int rows, int blocks,
-                          int n_groups, int max_chunks, hipStream_t st, float *amax_v = nullptr,
-                          int *amax_i = nullptr, bool group_tables = false,
-                          const void *w2 = nullptr, float *y2 = nullptr, bool fast = false,
-                          bool few = false);
-// Grouped (grp_expert set): sub_start holds 2 * (n_groups + 1) entries, the
-// chunk prefix sub_start[0..n_groups] and the twin prefix after it
-// (launch_moe_group's layout); group_tables: the GroupItem records follow
-// (written with the same max_chunks). act_q / act_d: the token-chunked
-// activations (q8k_wave.hpp). w2 / y2: a second matrix of the same shape on
-// the same activations, in the same launch. fast: the REDUCTION-tolerance
-// kernels (one float accumulator per output instead of the reference's eight
-// class sums; outputs within REDUCTION of dot_q6k_q8k, not bit-identical).
-// few: exact grouped calls (with group_tables) that leave most groups a token
-// or two.
+struct GroupItem;
+// Expert-grouped batched matvec (q6k_mv.hip) on activations in the token-chunked
+// layout (q8k_wave.hpp). records: launch_moe_group's, of n_groups experts and
+// max_chunks chunks; the output of the pair at sorted position i is row
+// pair_out[i] of y (nullptr: row i). Without records there is one group (expert
+// 0) of n_groups tokens in max_chunks chunks. w2 / y2: a second matrix of the
+// same shape on the same activations, in the same launch. fast: the
+// REDUCTION-tolerance kernels (one float accumulator per output instead of the
+// reference's eight class sums; outputs within REDUCTION of dot_q6k_q8k, not
+// bit-identical). few: exact grouped calls that leave most groups a token or two.
+int launch_q6k_mv_batched(const void *w, size_t expert_stride, const GroupItem *records,
+                          const int32_t *pair_out, const int8_t *act_q, const float *act_d, float *y,
+                          int ldy, int rows, int blocks, int n_groups, int max_chunks, hipStream_t st,
+                          float *amax_v = nullptr, int *amax_i = nullptr, const void *w2 = nullptr,
+                          float *y2 = nullptr, bool fast = false, bool few = false);
 
 // The REDUCTION GEMM of launch_q6k_mv_batched for many tokens per expert, on
 // moe_group's units of up to GROUP_WIDE_CHUNKS chunks (same sums, same bits).
@@ -133,7 +122,7 @@ bool q6k_wide_fits(int rows, int blocks);
 // Workgroups that a unit makes of these rows.
 int q6k_wide_groups(int rows, bool pair);
 int launch_q6k_mv_batched_wide(const void *w, const void *w2, size_t expert_stride,
-                               const int32_t *sub_start, const int32_t *pair_out,
+                               const GroupItem *records, const int32_t *pair_out,
                                const int8_t *act_q, const float *act_d, float *y, int rows,
                                int blocks, int n_groups, int max_chunks, hipStream_t st);
 // Up to three matrices with their own row counts (Q, K, V) against the same
@@ -174,13 +163,10 @@ int launch_swiglu_q8k(const float *gate, const float *up, float *act_out, int8_t
                       int16_t *bsums, int nblocks, hipStream_t st);
 int launch_swiglu_q8k_chunks(const float *gate, const float *up, int rows, int blocks,
                              const int32_t *slot_of, int8_t *cq, float *cd, hipStream_t st);
-// moe grouping (group.hip): counting sort of the (token, k) pairs by expert.
-// Outputs grp_* per expert, sub_start (prefix of ceil(count/16), then the
-// twin prefix of ceil(chunks/2): 2 * (n_expert + 1) entries; with
-// max_chunks > 0 then a GroupItem per chunk, per twin and per wide unit, from
-// group_items_offset(n_expert): group_table_size entries in all), for each
-// pair p = token * n_used + k its chunk slot slot_of_pair[p], and for each
-// sorted position its pair index pair_idx.
+// moe grouping (group.hip): counting sort of the (token, k) pairs by expert. For
+// each pair p = token * n_used + k its chunk slot slot_of_pair[p], for each sorted
+// position its pair index pair_idx, and a GroupItem per chunk, per twin and per
+// wide unit in records (group_records of them).
 // One work item of the expert-grouped batched kernels: a 16-token chunk, or a
 // twin (two consecutive chunks of one expert), with its group's fields.
 struct __attribute__((aligned(32))) GroupItem {
@@ -192,9 +178,6 @@ struct __attribute__((aligned(32))) GroupItem {
     int32_t twin2;   // twins: 1 when the second chunk exists; wide units: chunks
     int32_t pad0, pad1;
 };
-// The records start at this int32 offset of sub_start (32-byte aligned
-// when sub_start is).
-constexpr size_t group_items_offset(int n_expert) { return ((2 * (size_t)(n_expert + 1)) + 7) & ~(size_t)7; }
 // Wide units: up to this many consecutive chunks of one expert, and the
 // records (a multiple of 8) that any grouping into max_chunks chunks takes.
 // Where the routing leaves few units, they are shorter: 1, 2 or 4 chunks at
@@ -203,15 +186,12 @@ constexpr int GROUP_WIDE_CHUNKS = 8;
 constexpr int group_wide_units(int n_expert, int max_chunks) {
     return (max_chunks / GROUP_WIDE_CHUNKS + n_expert + 7) / 8 * 8;
 }
-// int32 entries of sub_start with its records
-constexpr size_t group_table_size(int n_expert, int max_chunks) {
-    return group_items_offset(n_expert) +
-           (2 * (size_t)max_chunks + group_wide_units(n_expert, max_chunks)) * sizeof(GroupItem) / 4;
+constexpr size_t group_records(int n_expert, int max_chunks) {
+    return 2 * (size_t)max_chunks + group_wide_units(n_expert, max_chunks);
 }
-int launch_moe_group(const int32_t *ids, int n_pairs, int n_used, int n_expert,
-                     int32_t *grp_expert, int32_t *grp_start, int32_t *grp_count,
-                     int32_t *sub_start, int32_t *slot_of_pair, int32_t *pair_idx,
-                     hipStream_t st, int max_chunks = 0, int wide_few = 0);
+int launch_moe_group(const int32_t *ids, int n_pairs, int n_expert, GroupItem *records,
+                     int32_t *slot_of_pair, int32_t *pair_idx, hipStream_t st, int max_chunks,
+                     int wide_few = 0);
 int launch_silu_mul(const float *gate, const float *up, float *out, int n, hipStream_t st);
 
 // norm.hip: CpuBackend::rms_norm (+ weight), bit-exact. rows of n; the

@@ -398,29 +398,24 @@ __global__ __launch_bounds__(256) void q6k_dequant_tiled(const uint8_t *w, int r
 // token) is the reference's, so every output is again bit-identical to
 // dot_q6k_q8k on that token's activation.
 //
-// Work: one wave per (group g, 16-token sub-tile st, 16-row tile t). A group
-// is one expert and a list of (activation index, output index) pairs; the LM
+// Work: one wave per (16-token chunk, or two, of one group; 16-row tile t). A
+// group is one expert and its run of sorted pairs (moe_group's records); the LM
 // head at batch 16 is one group of 16 tokens. Activations are read in the
-// class-major order written by the quantize kernels (byte 32 c + m of each
-// block holds weight 8 m + c).
+// token-chunked layout (q8k_wave.hpp).
 struct BatchParams {
     const uint8_t *w;
     size_t expert_stride;
-    const int32_t *grp_expert;   // [n_groups]
-    const int32_t *grp_start;    // first pair of the group
-    const int32_t *grp_count;    // pairs in the group
-    const int32_t *sub_start;    // prefix sum of ceil(count/16) over groups
     const int32_t *pair_out;     // output row of each sorted pair (nullptr: identity)
     const int8_t *act_q;         // token-chunked Q8_K quants (q8k_wave.hpp)
     const float *act_d;          // their scales
     float *y;                    // y[pair_out * ldy + row]
     float *amax_v;               // optional per-(token, tile) arg-max candidates
     int *amax_i;                 //   [token][tiles] (single group only)
-    int ldy, rows, tiles, blocks, n_groups;
-    int single_count;            // grp_expert == nullptr: one group, expert 0, this many tokens
-    const GroupItem *sub_info;   // optional: each chunk's / twin's record
-    const GroupItem *twin_info;  //   (launch_moe_group), else a binary search
-    const GroupItem *wide_info;  // units of up to WIDE_CHUNKS chunks (q6k_mv_batched_wide)
+    int ldy, rows, tiles, blocks;
+    int single_count;            // sub_info == nullptr: one group, expert 0, this many tokens
+    const GroupItem *sub_info;   // each chunk's record (launch_moe_group)
+    const GroupItem *twin_info;  // each twin's
+    const GroupItem *wide_info;  // each wide unit's (q6k_mv_batched_wide)
     // optional second matrix of the same shape on the same activations (gate
     // and up in one launch): items from items_per_mat on use w2 / y2
     const uint8_t *w2;
@@ -510,7 +505,7 @@ __device__ __forceinline__ void fold_digits(uint64_t codes, const FoldScales &f,
 }
 
 
-// The outputs of batched_tile's sums: y, and the tile's arg-max candidates.
+// The outputs of tile_block's sums: y, and the tile's arg-max candidates.
 template <int NC>
 __device__ __forceinline__ void batched_store(const BatchParams &p, const float (&sums)[NC][8][4], int lane,
                                               int t, int st0, int cnt, int start) {
@@ -615,228 +610,9 @@ __device__ __forceinline__ void tile_block(const TileRegs &r, const float (&adb)
     }
 }
 
-// The work of one wave on one 16-row tile t of expert `expert`'s weights
-// against NC consecutive 16-token chunks sub0.. of the token-chunked
-// activations (local chunk numbers st0.. inside the group of `cnt` pairs
-// starting at sorted position `start`). The weight codes are unpacked and
-// folded once per class and feed the MFMAs of all NC chunks, so a second
-// chunk costs only its MFMAs and its float epilogue.
-template <int NC, bool PF = false>
-__device__ __forceinline__ void batched_tile(const BatchParams &p, int lane, int t, int sub0,
-                                             int st0, int cnt, int start, int expert) {
-    const int n = lane & 15, s = lane >> 4;
-    const uint8_t *seg = p.w + (size_t)expert * p.expert_stride + (size_t)t * p.blocks * SEG_BYTES;
-    const size_t chunk_q = (size_t)p.blocks * CHUNK_BLOCK_BYTES, chunk_d = (size_t)p.blocks * CHUNK_TOKENS;
-    const int8_t *aq = p.act_q + (size_t)sub0 * chunk_q + 16 * lane;
-    const float *ad = p.act_d + (size_t)sub0 * chunk_d + n;
-
-    float sums[NC][8][4];
-#pragma unroll
-    for (int u = 0; u < NC; ++u)
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) sums[u][c][v] = 0.0f;
-
-    // one block's operands: the lane's weight words and its chunks' class
-    // planes and scales
-    struct Regs {
-        uint4 q0, q1, q2;
-        uint32_t scw;
-        uint2 dw;
-        float adb[NC];
-    };
-    auto load = [&](Regs &r, int b) {
-        const uint8_t *sg = seg + (size_t)b * SEG_BYTES;
-        r.q0 = *(const uint4 *)(sg + 16 * lane);
-        r.q1 = *(const uint4 *)(sg + SEG_PART + 16 * lane);
-        r.q2 = *(const uint4 *)(sg + 2 * SEG_PART + 16 * lane);
-        r.scw = *(const uint32_t *)(sg + SEG_SC + 4 * lane);
-        r.dw = *(const uint2 *)(sg + SEG_D + 8 * s);  // f16 d of rows 4s..4s+3
-#pragma unroll
-        for (int u = 0; u < NC; ++u) {
-            r.adb[u] = ad[u * chunk_d + (size_t)b * CHUNK_TOKENS];
-        }
-    };
-    // the class planes run BQ classes ahead of their MFMAs, across block
-    // boundaries (8 % BQ == 0, so a class keeps its ring slot); past the
-    // last block the loads re-read it, unused
-    constexpr int BQ = 2;
-    const int last = p.blocks - 1;
-    long act[BQ][NC];
-    auto aload = [&](int b, int c) {
-#pragma unroll
-        for (int u = 0; u < NC; ++u)
-            act[c % BQ][u] = *(const long *)(aq + u * chunk_q + (size_t)min(b, last) * CHUNK_BLOCK_BYTES +
-                                             1024 * (c >> 1) + 8 * (c & 1));
-    };
-    auto compute = [&](const Regs &r, int b) {
-        const uint32_t nib[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
-        const uint32_t hb[4] = {r.q2.x, r.q2.y, r.q2.z, r.q2.w};
-        const FoldScales fs = fold_scales(r.scw);
-        // f16(d) of the lane's 4 rows (D rows 4s..4s+3) times the token's scale
-        const float d4[4] = {f16_bits_to_f32((uint16_t)(r.dw.x & 0xFFFF)),
-                             f16_bits_to_f32((uint16_t)(r.dw.x >> 16)),
-                             f16_bits_to_f32((uint16_t)(r.dw.y & 0xFFFF)),
-                             f16_bits_to_f32((uint16_t)(r.dw.y >> 16))};
-        float dd[NC][4];
-#pragma unroll
-        for (int u = 0; u < NC; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) dd[u][v] = d4[v] * r.adb[u];
-        const v4i zero = {0, 0, 0, 0};
-        // software-pipelined by one class: the MFMAs of class c+1 are issued
-        // before the epilogue of class c reads its results
-        v4i dh[2][NC], dl[2][NC];
-        {
-            long a_lo, a_hi;
-            fold_digits((uint64_t)unpack_codes(nib, hb, 0), fs, a_lo, a_hi);
-#pragma unroll
-            for (int u = 0; u < NC; ++u) {
-                dh[0][u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, act[0][u], zero, 0, 0, 0);
-                dl[0][u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, act[0][u], zero, 0, 0, 0);
-            }
-            aload(BQ < 8 ? b : b + 1, BQ % 8);
-        }
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if (c + 1 < 8) {
-                long a_lo, a_hi;
-                fold_digits((uint64_t)unpack_codes(nib, hb, c + 1), fs, a_lo, a_hi);
-#pragma unroll
-                for (int u = 0; u < NC; ++u) {
-                    dh[(c + 1) & 1][u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, act[(c + 1) % BQ][u], zero, 0, 0, 0);
-                    dl[(c + 1) & 1][u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, act[(c + 1) % BQ][u], zero, 0, 0, 0);
-                }
-                aload(c + 1 + BQ < 8 ? b : b + 1, (c + 1 + BQ) % 8);
-            }
-#pragma unroll
-            for (int u = 0; u < NC; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int aux = dh[c & 1][u][v] * 256 + dl[c & 1][u][v];
-                    sums[u][c][v] = sums[u][c][v] + dd[u][v] * (float)aux;
-                }
-        }
-    };
-    if constexpr (PF) {
-        // two register sets in ping-pong: the next block's loads are in
-        // flight while the current block is computed. The loads are
-        // unconditional (past the last block they re-read it, unused), so
-        // the compiler waits for each block's own loads only.
-        Regs ra, rb;
-        load(ra, 0);
-#pragma unroll
-        for (int c = 0; c < BQ; ++c) aload(0, c);
-        for (int b = 0; b < p.blocks; b += 2) {
-            load(rb, min(b + 1, last));
-            compute(ra, b);
-            if (b + 1 >= p.blocks) break;
-            load(ra, min(b + 2, last));
-            compute(rb, b + 1);
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < BQ; ++c) aload(0, c);
-        for (int b = 0; b < p.blocks; ++b) {
-            Regs r;
-            load(r, b);
-            compute(r, b);
-        }
-    }
-    batched_store<NC>(p, sums, lane, t, st0, cnt, start);
-}
-
-// One wave per (group, 16-token chunk, 16-row tile). The chunk index is the
-// global sub-tile number, which is also where the activations of its 16
-// tokens sit in the token-chunked layout.
-__global__ __launch_bounds__(256) void q6k_mv_batched(BatchParams pk) {
-    const int lane = threadIdx.x & 63;
-    BatchParams p;
-    const int item = batch_item(pk, p);
-    if (item >= p.items_per_mat) return;  // the grid's rounding to whole workgroups
-    const int t = item % p.tiles;
-    const int sub = item / p.tiles;
-    int st = sub, cnt, start = 0, expert = 0;
-    if (p.grp_expert) {
-        // find the group whose chunk range holds `sub` (sub_start has
-        // n_groups + 1 entries)
-        if (p.sub_info) {
-            const GroupItem it = p.sub_info[sub];  // expert -1: a spare item
-            if (it.expert < 0) return;
-            st = it.st;
-            cnt = it.count;
-            start = it.start;
-            expert = it.expert;
-        } else {
-            if (sub >= p.sub_start[p.n_groups]) return;
-            int lo = 0, hi = p.n_groups;
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (p.sub_start[mid] <= sub) lo = mid; else hi = mid;
-            }
-            st = sub - p.sub_start[lo];
-            cnt = p.grp_count[lo];
-            start = p.grp_start[lo];
-            expert = p.grp_expert[lo];
-        }
-    } else {
-        cnt = p.single_count;
-        if (sub >= (cnt + 15) / 16) return;
-    }
-    batched_tile<1, true>(p, lane, t, sub, st, cnt, start, expert);
-}
-
-// One wave per (group, twin, 16-row tile): a twin is two consecutive chunks
-// of one group (the group's last twin holds one chunk when its chunk count is
-// odd). twin_start = sub_start + n_groups + 1 is the prefix sum of
-// ceil(chunks/2) over the groups. The shared fold takes the VALU work of a
-// twin from 2 x 325 to 460 instructions per block; the register budget is
-// capped at 3 waves per SIMD (168 VGPRs, a few spilled), which measured 20%
-// faster than the uncapped 178 VGPRs at 2 waves and 5% faster than one chunk
-// per wave.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void q6k_mv_batched_twin(BatchParams pk) {
-    const int lane = threadIdx.x & 63;
-    BatchParams p;
-    const int item = batch_item(pk, p);
-    if (item >= p.items_per_mat) return;  // the grid's rounding to whole workgroups
-    const int t = item % p.tiles;
-    const int tw = item / p.tiles;
-    const int32_t *twin_start = p.sub_start + p.n_groups + 1;
-    int st, sub, cnt, start, expert;
-    bool two;
-    if (p.twin_info) {
-        const GroupItem it = p.twin_info[tw];  // expert -1: a spare item
-        if (it.expert < 0) return;
-        st = it.st;
-        sub = it.sub;
-        cnt = it.count;
-        start = it.start;
-        expert = it.expert;
-        two = it.twin2 != 0;
-    } else {
-        if (tw >= twin_start[p.n_groups]) return;
-        int lo = 0, hi = p.n_groups;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (twin_start[mid] <= tw) lo = mid; else hi = mid;
-        }
-        st = 2 * (tw - twin_start[lo]);
-        sub = p.sub_start[lo] + st;
-        cnt = p.grp_count[lo];
-        start = p.grp_start[lo];
-        expert = p.grp_expert[lo];
-        two = sub + 1 < p.sub_start[lo + 1];
-    }
-    if (two)
-        batched_tile<2>(p, lane, t, sub, st, cnt, start, expert);
-    else
-        batched_tile<1>(p, lane, t, sub, st, cnt, start, expert);
-}
-
 // ---- REDUCTION-tolerance batched kernels (LLAMD_HIP_REDUCTION) ----------------
 //
-// The same operands, digits and MFMAs as batched_tile, but the MFMAs of all 8
+// The same operands and digits as tile_block, but the MFMAs of all 8
 // classes of a block accumulate into one pair of digit accumulators: the
 // block's integer dot sum_c aux32[c] is exact in int32 (|.| < 2^27), and the
 // float epilogue is one convert and one fused multiply-add per (row, token,
@@ -847,11 +623,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // K is split over KS waves of one workgroup (a shorter dependent chain of
 // block loads per wave, KS times the waves in flight), met in LDS.
 
-// The lane's partial sums (4 rows x NC chunks) over blocks [b0, b1) of tile t.
-// The dynamic LDS of the LDSA kernels below.
+// The dynamic LDS of the staged kernels below.
 extern __shared__ uint4 g_act_lds[];
 
-// LDSA: the chunk's quants are read from g_act_lds (same layout).
 // The digit operands of the 64-deep MFMA of classes 2 P and 2 P + 1.
 __device__ __forceinline__ void fold_pair(const uint32_t nib[8], const uint32_t hb[4], int P,
                                           const FoldScales &fs, v4i &lo, v4i &hi) {
@@ -862,6 +636,8 @@ __device__ __forceinline__ void fold_pair(const uint32_t nib[8], const uint32_t 
     hi = v4i{(int)h[0], (int)(h[0] >> 32), (int)h[1], (int)(h[1] >> 32)};
 }
 
+// The lane's partial sums (4 rows x NC chunks) over blocks [b0, b1) of tile t.
+// LDSA: the chunk's quants are read from g_act_lds (same layout).
 template <int NC, bool LDSA = false>
 __device__ __forceinline__ void fast_tile_range(const BatchParams &p, int lane, int t, int sub0,
                                                 int expert, int b0, int b1, float acc[2][4]) {
@@ -953,7 +729,7 @@ __device__ __forceinline__ void fast_tile_range(const BatchParams &p, int lane, 
 
 // KS waves per work item (4 / KS items per workgroup). TWIN: the items are
 // twins (moe_group's twin records), else 16-token chunks (chunk records, or
-// the single group of grp_expert == nullptr).
+// the single group).
 // LDSA: one 16-token chunk for the whole grid (the LM head at batch <= 16):
 // each workgroup first copies the chunk's quants (blocks x 4 KiB, dynamic
 // LDS) once, so the class-plane loads of every block read LDS instead of
@@ -976,7 +752,7 @@ __global__ __launch_bounds__(256) void q6k_mv_batched_fast(BatchParams pk) {
     if (live) {
         t = item % p.tiles;
         const int unit = item / p.tiles;
-        if (p.grp_expert) {
+        if (p.sub_info) {
             const GroupItem it = TWIN ? p.twin_info[unit] : p.sub_info[unit];  // expert -1: spare
             live = it.expert >= 0;
             st = it.st;
@@ -1073,7 +849,7 @@ using lds_ptr = __attribute__((address_space(3))) void *;
 // sequences): a workgroup per (chunk, tile), wave P on classes 2P and 2P + 1
 // alone. Each class's sum stays with one wave, block after block, and one
 // thread per output adds the eight in class order, so the bits are those of
-// q6k_mv_batched; the chip gets four times the waves, each with a quarter
+// q6k_mv_batched_staged; the chip gets four times the waves, each with a quarter
 // of the chain (QKV of 5120 x 2048 on 5 sequences: 16.5 -> 14.4 us a call, norm and
 // quants included).
 __global__ __launch_bounds__(256) void q6k_mv_batched_classes(BatchParams pk) {
@@ -2147,31 +1923,24 @@ int launch_one_group(BatchParams &p, int chunks, long items, hipStream_t st) {
 }
 }  // namespace
 
-int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *grp_expert,
-                          const int32_t *grp_start, const int32_t *grp_count,
-                          const int32_t *sub_start, const int32_t *pair_out, const int8_t *act_q,
-                          const float *act_d, float *y, int ldy, int rows, int blocks,
-                          int n_groups, int max_chunks, hipStream_t st, float *amax_v,
-                          int *amax_i, bool group_tables, const void *w2, float *y2, bool fast, bool few) {
-    if (amax_v && grp_expert) return -1;
+int launch_q6k_mv_batched(const void *w, size_t expert_stride, const GroupItem *records,
+                          const int32_t *pair_out, const int8_t *act_q, const float *act_d, float *y,
+                          int ldy, int rows, int blocks, int n_groups, int max_chunks, hipStream_t st,
+                          float *amax_v, int *amax_i, const void *w2, float *y2, bool fast, bool few) {
+    if (amax_v && records) return -1;
     // every item of the grids below indexes a record below max_chunks when
     // max_chunks >= n_groups (twins: ceil((max_chunks + n_groups) / 2) items)
-    if (group_tables && (!grp_expert || max_chunks < n_groups || max_chunks <= 0)) return -1;
-    BatchParams p;
-    p.n_segs = 0;
+    if (records && max_chunks < n_groups) return -1;
+    if (max_chunks <= 0 || rows <= 0) return 0;
+    BatchParams p = {};
     if (w2 && (!y2 || amax_v)) return -1;
     p.w2 = (const uint8_t *)w2;
     p.y2 = y2;
-    p.sub_info = group_tables ? (const GroupItem *)(sub_start + group_items_offset(n_groups)) : nullptr;
-    p.twin_info = group_tables ? p.sub_info + max_chunks : nullptr;
-    p.wide_info = group_tables ? p.twin_info + max_chunks : nullptr;
-    p.single_count = n_groups;  // only read when grp_expert == nullptr
+    p.sub_info = records;
+    p.twin_info = records ? records + max_chunks : nullptr;
+    p.single_count = n_groups;  // only read without records
     p.w = (const uint8_t *)w;
     p.expert_stride = expert_stride;
-    p.grp_expert = grp_expert;
-    p.grp_start = grp_start;
-    p.grp_count = grp_count;
-    p.sub_start = sub_start;
     p.pair_out = pair_out;
     p.act_q = act_q;
     p.act_d = act_d;
@@ -2182,25 +1951,22 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
     p.rows = rows;
     p.tiles = (rows + TILE_ROWS - 1) / TILE_ROWS;
     p.blocks = blocks;
-    p.n_groups = n_groups;
+    // twins: sum of ceil(ch/2) <= (sum of ch + n_groups) / 2
+    const bool twin = records && g_tune_batched_twin && (fast || !few);
+    const long items = (long)p.tiles * (twin ? (max_chunks + n_groups + 1) / 2 : max_chunks);
+    const long all = w2 ? 2 * items : items;
+    p.items_per_mat = (int)items;
     if (fast) {
         // K split over ks waves (tune key fast_ks): one measured best on
         // MI355X for both the prefill and the LM head shapes
         const int ks = g_tune_fast_ks ? g_tune_fast_ks : 1;
-        const bool twin = grp_expert && g_tune_batched_twin;
-        if (grp_expert && !group_tables) return -1;
-        const long units = twin ? (max_chunks + n_groups + 1) / 2 : max_chunks;
-        const long items = (long)p.tiles * units;
-        if (items <= 0) return 0;
-        p.items_per_mat = (int)items;
-        const long all = w2 ? 2 * items : items;
         const unsigned grid = (unsigned)((all * ks + 3) / 4);
         const size_t lds = (size_t)blocks * CHUNK_BLOCK_BYTES;
-        if (grp_expert && ks == 1 && p.tiles % 4 == 0 && g_tune_fast_lds) {
+        if (records && ks == 1 && p.tiles % 4 == 0 && g_tune_fast_lds) {
             const size_t slds = (size_t)2 * (twin ? 2 : 1) * CHUNK_BLOCK_BYTES;
             if (twin) hipLaunchKernelGGL(q6k_mv_batched_fast_staged<true>, dim3(grid), dim3(256), slds, st, p);
             else hipLaunchKernelGGL(q6k_mv_batched_fast_staged<false>, dim3(grid), dim3(256), slds, st, p);
-        } else if (!grp_expert && n_groups <= CHUNK_TOKENS && lds <= 65536 && g_tune_fast_lds) {
+        } else if (!records && n_groups <= CHUNK_TOKENS && lds <= 65536 && g_tune_fast_lds) {
             if (ks == 4) hipLaunchKernelGGL((q6k_mv_batched_fast<4, false, true>), dim3(grid), dim3(256), lds, st, p);
             else if (ks == 2) hipLaunchKernelGGL((q6k_mv_batched_fast<2, false, true>), dim3(grid), dim3(256), lds, st, p);
             else hipLaunchKernelGGL((q6k_mv_batched_fast<1, false, true>), dim3(grid), dim3(256), lds, st, p);
@@ -2212,30 +1978,11 @@ int launch_q6k_mv_batched(const void *w, size_t expert_stride, const int32_t *gr
         else hipLaunchKernelGGL((q6k_mv_batched_fast<1, false>), dim3(grid), dim3(256), 0, st, p);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
-    if (group_tables && few && g_tune_batched_twin && (rows + TILE_ROWS - 1) / TILE_ROWS % 4 == 0) {
-        const long items = (long)p.tiles * max_chunks;
-        p.items_per_mat = (int)items;
-        hipLaunchKernelGGL(q6k_mv_batched_few, dim3((unsigned)((w2 ? 2 * items : items) / 4)), dim3(256),
-                           2 * CHUNK_BLOCK_BYTES, st, p);
-        return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
-    if (grp_expert && g_tune_batched_twin) {
-        // twins: sum of ceil(ch/2) <= (sum of ch + n_groups) / 2
-        const long items = (long)p.tiles * ((max_chunks + n_groups + 1) / 2);
-        if (items <= 0) return 0;
-        p.items_per_mat = (int)items;
-        const long all = w2 ? 2 * items : items;
-        if (group_tables && p.tiles % 4 == 0)
-            hipLaunchKernelGGL(q6k_mv_batched_twin_staged, dim3((unsigned)(all / 4)), dim3(256), 4 * CHUNK_BLOCK_BYTES, st, p);
-        else hipLaunchKernelGGL(q6k_mv_batched_twin, dim3((unsigned)((all + 3) / 4)), dim3(256), 0, st, p);
-        return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
-    const long items = (long)p.tiles * max_chunks;
-    if (items <= 0) return 0;
-    p.items_per_mat = (int)items;
-    const long all = w2 ? 2 * items : items;
-    if (!grp_expert) return launch_one_group(p, max_chunks, all, st);
-    hipLaunchKernelGGL(q6k_mv_batched, dim3((unsigned)((all + 3) / 4)), dim3(256), 0, st, p);
+    if (!records) return launch_one_group(p, max_chunks, all, st);
+    // (a layer's rows are multiples of 256)
+    if (p.tiles % 4) return -1;
+    if (twin) hipLaunchKernelGGL(q6k_mv_batched_twin_staged, dim3((unsigned)(all / 4)), dim3(256), 4 * CHUNK_BLOCK_BYTES, st, p);
+    else hipLaunchKernelGGL(q6k_mv_batched_few, dim3((unsigned)(all / 4)), dim3(256), 2 * CHUNK_BLOCK_BYTES, st, p);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -2247,7 +1994,7 @@ int q6k_wide_groups(int rows, bool pair) {
 bool q6k_wide_fits(int rows, int blocks) { return rows % TILE_ROWS == 0 && blocks <= WIDE_MAX_BLOCKS; }
 
 int launch_q6k_mv_batched_wide(const void *w, const void *w2, size_t expert_stride,
-                               const int32_t *sub_start, const int32_t *pair_out,
+                               const GroupItem *records, const int32_t *pair_out,
                                const int8_t *act_q, const float *act_d, float *y, int rows,
                                int blocks, int n_groups, int max_chunks, hipStream_t st) {
     if (!q6k_wide_fits(rows, blocks) || (uintptr_t)y % 16 || max_chunks <= 0) return -1;
@@ -2255,7 +2002,7 @@ int launch_q6k_mv_batched_wide(const void *w, const void *w2, size_t expert_stri
     p.w = (const uint8_t *)w;
     p.w2 = (const uint8_t *)w2;
     p.expert_stride = expert_stride;
-    p.wide_info = (const GroupItem *)(sub_start + group_items_offset(n_groups)) + 2 * (size_t)max_chunks;
+    p.wide_info = records + 2 * (size_t)max_chunks;
     p.pair_out = pair_out;
     p.act_q = act_q;
     p.act_d = act_d;
