@@ -433,10 +433,15 @@ struct BatchParams {
 };
 
 // The work item of this wave and the parameters it runs with: the second
-// matrix's items are the first's, offset by items_per_mat.
+// matrix's items are the first's, offset by items_per_mat. The item is the same
+// for the whole wave, so its addresses stay in SGPRs (twins 168 -> 154 registers);
+// SEGS false: grouped calls, which have no segments to choose from. Together 512
+// tokens 258.6 -> 248.6 us a call, 45 104.7 -> 102.3, a layer of 16 sequences
+// 109.4 -> 107.2.
+template <bool SEGS>
 __device__ __forceinline__ int batch_item(const BatchParams &p, BatchParams &q, int item) {
     q = p;
-    if (p.n_segs > 0) {
+    if (SEGS && p.n_segs > 0) {
         // the item's segment, chosen with scalar selects
         BatchParams::Seg sg = p.segs[0];
         if (p.n_segs > 1 && item >= p.segs[1].first) sg = p.segs[1];
@@ -454,9 +459,6 @@ __device__ __forceinline__ int batch_item(const BatchParams &p, BatchParams &q, 
         q.y = p.y2;
     }
     return item;
-}
-__device__ __forceinline__ int batch_item(const BatchParams &p, BatchParams &q) {
-    return batch_item(p, q, (int)blockIdx.x * 4 + (threadIdx.x >> 6));
 }
 
 typedef short s16x2 __attribute__((ext_vector_type(2)));
@@ -850,13 +852,12 @@ using lds_ptr = __attribute__((address_space(3))) void *;
 // alone. Each class's sum stays with one wave, block after block, and one
 // thread per output adds the eight in class order, so the bits are those of
 // q6k_mv_batched_staged; the chip gets four times the waves, each with a quarter
-// of the chain (QKV of 5120 x 2048 on 5 sequences: 16.5 -> 14.4 us a call, norm and
-// quants included).
+// of the chain (launch_one_group has the figures).
 __global__ __launch_bounds__(256) void q6k_mv_batched_classes(BatchParams pk) {
     __shared__ float part[8][4][64];  // [class][v][lane]
     const int lane = threadIdx.x & 63, P = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     BatchParams p;
-    const int item = batch_item(pk, p, (int)blockIdx.x);
+    const int item = batch_item<true>(pk, p, (int)blockIdx.x);
     const int t = item % p.tiles, chunk = item / p.tiles;
     if (CHUNK_TOKENS * chunk >= p.single_count) return;
     const uint8_t *seg = p.w + (size_t)t * p.blocks * SEG_BYTES;
@@ -1108,7 +1109,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     BatchParams p;
-    const int item = batch_item(pk, p);
+    const int item = batch_item<false>(pk, p, (int)blockIdx.x * 4 + wave);
     if (item >= p.items_per_mat) return;
     const GroupItem it = p.twin_info[item / p.tiles];
     if (it.expert < 0) return;
@@ -1129,7 +1130,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     BatchParams p;
-    const int item = batch_item(pk, p);
+    const int item = batch_item<true>(pk, p, (int)blockIdx.x * 4 + wave);
     const int chunk = item / staged_slots(p.tiles), t = item % staged_slots(p.tiles);
     if (CHUNK_TOKENS * chunk >= p.single_count) return;
     const GroupItem it = {0, chunk, chunk, t < p.tiles ? p.single_count : 0, 0, 0, 0, 0};
@@ -1141,7 +1142,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     BatchParams p;
-    const int item = batch_item(pk, p);
+    const int item = batch_item<false>(pk, p, (int)blockIdx.x * 4 + wave);
     if (item >= p.items_per_mat) return;
     const GroupItem it = p.sub_info[item / p.tiles];
     if (it.expert < 0) return;
@@ -1903,7 +1904,7 @@ namespace {
 // chunks in all.
 int launch_one_group(BatchParams &p, int chunks, long items, hipStream_t st) {
     // half a wave per SIMD or less (us per call with the norm and the quants, a
-    // wave per item -> four: 320 items 15.9 -> 14.4, 640 16.3 -> 16.8)
+    // wave per item -> four: 320 items (5120 x 2048) 15.9 -> 14.4, 640 16.3 -> 16.8)
     if (items <= 512 && !p.amax_v) {
         hipLaunchKernelGGL(q6k_mv_batched_classes, dim3((unsigned)items), dim3(256), 0, st, p);
         return hipGetLastError() == hipSuccess ? 0 : -1;
