@@ -483,7 +483,7 @@ struct AttArgs {
     float *scores;            // [nseq][n_head][cap]
     float *out;               // [nseq][n_head * HD]
     size_t seq_stride;        // floats between two sequences' caches
-    int pos_stride, n_kv_fixed, n_head, n_head_kv, cap, fuse, grid_x;
+    int pos_stride, n_kv_fixed, n_head, n_head_kv, cap, fuse, grid_y;
     float scale;
 };
 
@@ -506,13 +506,13 @@ __global__ __launch_bounds__(64 * AS_MAX_GROUP) void attend_scores(AttArgs a) {
     const int group = a.n_head / a.n_head_kv, nt = 64 * group;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int g = blockIdx.y, s = blockIdx.z;
+    const int g = blockIdx.x % a.n_head_kv, s = blockIdx.x / a.n_head_kv;
     const int n_kv = att_n_kv(a, s), kv_dim = a.n_head_kv * HD;
     if (n_kv <= a.fuse || n_kv > a.cap) return;
     const int head = s * a.n_head + g * group + wave;
     const att_cptr q = (att_cptr)(a.q + (size_t)head * HD);
     const float *kc = a.kc + (size_t)s * a.seq_stride + (size_t)g * HD;
-    for (int t0 = blockIdx.x * AS_POS; t0 < n_kv; t0 += a.grid_x * AS_POS) {
+    for (int t0 = blockIdx.y * AS_POS; t0 < n_kv; t0 += a.grid_y * AS_POS) {
         const int np = min(AS_POS, n_kv - t0);
         __syncthreads();  // the previous block's rows are read
         for (int i0 = tid; i0 < np * (HD / 4); i0 += 4 * nt) {
@@ -522,7 +522,7 @@ __global__ __launch_bounds__(64 * AS_MAX_GROUP) void attend_scores(AttArgs a) {
                 const int i = i0 + k * nt, t = min(i / (HD / 4), np - 1);
                 r[k] = *(const att_f4 *)(kc + (size_t)(t0 + t) * kv_dim + 4 * (i % (HD / 4)));
             }
-            if (t0 == (int)blockIdx.x * AS_POS && i0 == tid) att_touch<HD>(q);
+            if (t0 == (int)blockIdx.y * AS_POS && i0 == tid) att_touch<HD>(q);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int i = i0 + k * nt, t = i / (HD / 4);
@@ -1034,8 +1034,11 @@ int launch_attend_split(const float *q, const float *kc, const float *vc, const 
     // Slices of up to 1024 may have 32 a CU, one round (13 of 1000 28.8, 29.3 with 512).
     const int blocks = (expect + AS_POS - 1) / AS_POS, pairs = n_head_kv * nseq;
     const int most = std::min(2048, (blocks <= 16 ? 8192 : 4096) / (n_head / n_head_kv));
-    a.grid_x = std::min(blocks, (most + pairs - 1) / pairs);
-    const dim3 grid(a.grid_x, n_head_kv, nseq), block(64 * (n_head / n_head_kv));
+    a.grid_y = std::min(blocks, (most + pairs - 1) / pairs);
+    // kv heads and sequences first: where only the first blocks find positions,
+    // their workgroups are on all XCDs, not on one or two (16 of 80 in slices of
+    // 2048, 16 query / 8 kv heads: 18.0, 9.4; 13 of 1000 28.7, 28.0)
+    const dim3 grid(pairs, a.grid_y), block(64 * (n_head / n_head_kv));
     if (hd == 128) hipLaunchKernelGGL(attend_scores<128>, grid, block, 0, st, a);
     else hipLaunchKernelGGL(attend_scores<64>, grid, block, 0, st, a);
     if (hipGetLastError() != hipSuccess) return -1;
