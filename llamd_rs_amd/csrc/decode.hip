@@ -474,6 +474,7 @@ __global__ __launch_bounds__(512) void attend_fused(
 constexpr int AS_POS = 64;          // positions per block of attend_scores
 constexpr int AS_MAX_GROUP = 16;    // query heads per kv head
 constexpr int ATT_SERIAL = 320;     // e_t that one lane adds
+constexpr int ATT_FEW = 56;         // positions that one wave takes (att_few)
 
 typedef const __attribute__((address_space(4))) float *att_cptr;
 
@@ -652,6 +653,54 @@ __device__ __forceinline__ float att_sum_serial(const float *lg, int n) {
     return sum;
 }
 
+// A sequence of up to ATT_FEW positions, without chunks: wave 0 takes a position
+// a lane; the DS / 64 waves after it, which fold, have the V rows in flight
+// meanwhile. (us a call, with chunks and without, 32 query / 4 kv heads: one
+// sequence of 1 position 5.3, 4.0; of 20 5.5, 4.2; of 48 5.7, 4.8; 32 of 20 13.7,
+// 9.3. From about 56 on a wave that reads the K rows by itself is behind: 16 of 64
+// 6.8, 7.4.)
+template <int HD, int DS>
+__device__ __forceinline__ void att_few(const float *q, const float *kc, const float *vc, int kv_dim,
+                                        int n_kv, float scale, float *lg, const uint64_t *tab, float *out) {
+    constexpr int A = 8;
+    static_assert(ATT_FEW <= 64 && ATT_FEW % A == 0, "a lane per position");
+    const int lane = threadIdx.x & 63, d = (int)threadIdx.x - 64;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const bool folds = wave > 0 && wave <= DS / 64;
+    float v[ATT_FEW], l = -INFINITY, mx = 0.0f;
+    if (folds) {
+#pragma unroll
+        for (int t0 = 0; t0 < ATT_FEW; t0 += A)
+            if (t0 < n_kv)  // (rows past the last re-read it, unused)
+#pragma unroll
+                for (int t = t0; t < t0 + A; ++t) v[t] = vc[(size_t)min(t, n_kv - 1) * kv_dim + d];
+    } else if (wave == 0) {
+        l = att_logit<HD>(q, kc + (size_t)min(lane, n_kv - 1) * kv_dim, scale);
+        // f32::max fold: NaN ignoring, order free (the last row taken again changes nothing)
+        mx = wave_reduce(l, -INFINITY, [](float x, float y) { return fmaxf(x, y); });
+    }
+    __syncthreads();  // tab
+    if (wave == 0) {
+        const float e = expf_ref_tab(l - mx, tab);
+        float sum = 0.0f;
+        for (int t = 0; t < n_kv; ++t)
+            sum = sum + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), t));
+        lg[lane] = e * __fdiv_rn(1.0f, sum);
+    }
+    __syncthreads();
+    if (!folds) return;
+    float acc = 0.0f;
+#pragma unroll
+    for (int t0 = 0; t0 < ATT_FEW; t0 += A)
+        if (t0 < n_kv)
+#pragma unroll
+            for (int t = t0; t < t0 + A; ++t) {
+                const float w = lg[t] * v[t];
+                acc = t < n_kv ? acc + w : acc;
+            }
+    out[d] = acc;
+}
+
 // The logits of every position into lg, from K rows staged 64 * TILES at a
 // time in `ks` (16-byte units of row t at unit u ^ t: conflict-free reads of one
 // unit by 64 rows); returns this thread's share of their max.
@@ -713,7 +762,9 @@ constexpr int am_threads = WIDE ? 64 * (1 + (NP + 2) / 3 * 3 + (NP - 1) / 3) : D
 template <int DS, int NP, bool WIDE>
 constexpr int am_chunk = (WIDE ? 1 : 2) * 1024 * NP / DS;
 
-template <int HD, int DS, int NP, bool WIDE, int TILES>
+// ONE: forms the logits of any number of positions; else attend_scores has formed
+// those of more than a.fuse.
+template <int HD, int DS, int NP, bool WIDE, int TILES, bool ONE>
 __global__ __launch_bounds__((am_threads<DS, NP, WIDE>)) void attend_mix(AttArgs a) {
     constexpr int NF = DS / 64, NT = am_threads<DS, NP, WIDE>, NW = NT / 64;
     constexpr int CH = am_chunk<DS, NP, WIDE>, HALF = CH / 2, D4 = DS / 4;
@@ -732,7 +783,8 @@ __global__ __launch_bounds__((am_threads<DS, NP, WIDE>)) void attend_mix(AttArgs
     constexpr int SL = HD / DS;
     const int g = blockIdx.x % a.n_head_kv, r = blockIdx.x / a.n_head_kv;
     const int h = g * (a.n_head / a.n_head_kv) + r / SL, sd = (r % SL) * DS, s = blockIdx.y;
-    const int kv_dim = a.n_head_kv * HD, n_kv = att_n_kv(a, s);
+    const int kv_dim = a.n_head_kv * HD;
+    int n_kv = att_n_kv(a, s);
     const float *q = a.q + ((size_t)s * a.n_head + h) * HD;
     const float *kc = a.kc + (size_t)s * a.seq_stride + (size_t)g * HD;
     const float *vc = a.vc + (size_t)s * a.seq_stride + (size_t)g * HD + sd;
@@ -748,6 +800,13 @@ __global__ __launch_bounds__((am_threads<DS, NP, WIDE>)) void attend_mix(AttArgs
         att_beyond_cap<HD, DS, NT>(a, q, kc, vc, kv_dim, n_kv, lg, red, tab, out);
         return;
     }
+    if (n_kv <= ATT_FEW) {
+        att_few<HD, DS>(q, kc, vc, kv_dim, n_kv, a.scale, lg, tab, out);
+        return;
+    }
+    // (the loops of this form fold slower where the compiler knows n_kv > ATT_FEW:
+    // 13 sequences of 1000 30.2 us, 28.0)
+    if constexpr (!WIDE && !ONE) asm volatile("" : "+s"(n_kv));
     const int nc = (n_kv + CH - 1) / CH;
     // a producer thread's piece of a chunk: positions 4 t4 .. 4 t4 + 3, dimensions
     // 4 d4 .. 4 d4 + 3
@@ -776,7 +835,7 @@ __global__ __launch_bounds__((am_threads<DS, NP, WIDE>)) void attend_mix(AttArgs
     }
     // the logits and their max (f32::max fold: NaN ignoring, order free)
     float mx = -INFINITY;
-    if (n_kv <= a.fuse) {
+    if (ONE || n_kv <= a.fuse) {
         mx = att_logits_here<HD, NT, TILES>(q, kc, kv_dim, n_kv, a.scale, lg, buf);
     } else {
         const float *sc = a.scores + ((size_t)s * a.n_head + h) * a.cap;
@@ -961,15 +1020,15 @@ size_t split_lds(int cap, int hd, int ds, int chunk, int tiles) {
     return (size_t)(cap + 127) / 128 * 128 * 4 + std::max(2 * chunk * ds * 4, tiles * 64 * hd * 4);
 }
 
-template <int HD, int DS, int NP, bool WIDE, int TILES>
+template <int HD, int DS, int NP, bool WIDE, int TILES, bool ONE = false>
 int launch_mix(const AttArgs &a, int nseq, hipStream_t st) {
     constexpr int CH = am_chunk<DS, NP, WIDE>;
     // the largest cache's dynamic LDS, allowed once per kernel
-    static const hipError_t ok = hipFuncSetAttribute((const void *)attend_mix<HD, DS, NP, WIDE, TILES>,
+    static const hipError_t ok = hipFuncSetAttribute((const void *)attend_mix<HD, DS, NP, WIDE, TILES, ONE>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize,
                                                      (int)split_lds(ATT_MAX_KV, HD, DS, CH, TILES));
     if (ok != hipSuccess) return -1;
-    hipLaunchKernelGGL((attend_mix<HD, DS, NP, WIDE, TILES>), dim3(a.n_head * (HD / DS), nseq),
+    hipLaunchKernelGGL((attend_mix<HD, DS, NP, WIDE, TILES, ONE>), dim3(a.n_head * (HD / DS), nseq),
                        dim3(am_threads<DS, NP, WIDE>), split_lds(a.cap, HD, DS, CH, TILES), st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -1020,10 +1079,9 @@ int launch_attend_split(const float *q, const float *kc, const float *vc, const 
     if (expect <= ATT_ONE_LAUNCH) {
         // short caches: one launch of small workgroups that form the logits
         // themselves (at 300 positions the second launch already pays)
-        a.fuse = cap;
-        if (hd == 64) return launch_mix<64, 64, 4, false, 2>(a, nseq, st);
-        return heads <= 128 ? launch_mix<128, 64, 4, false, 2>(a, nseq, st)
-                            : launch_mix<128, 128, 4, false, 1>(a, nseq, st);
+        if (hd == 64) return launch_mix<64, 64, 4, false, 2, true>(a, nseq, st);
+        return heads <= 128 ? launch_mix<128, 64, 4, false, 2, true>(a, nseq, st)
+                            : launch_mix<128, 128, 4, false, 1, true>(a, nseq, st);
     }
     a.fuse = 64;
     // 16 waves a CU (at most 2048 workgroups), which take several blocks each

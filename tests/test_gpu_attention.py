@@ -34,7 +34,7 @@ def run_one(gpu, q, kc, vc, n_head, n_head_kv, hd, n_kv, max_kv=None):
 
 
 @pytest.mark.parametrize("n_head,n_head_kv,hd,lengths", [
-    (32, 4, 128, (1, 8, 20, 31, 64, 65, 96, 97, 129, 160, 161, 256, 257, 352, 1000, 4100)),
+    (32, 4, 128, (1, 8, 9, 20, 31, 33, 55, 56, 57, 64, 65, 96, 97, 129, 160, 161, 256, 257, 352, 1000, 4100)),
     (8, 1, 128, (6144, 6145, 6657, 8193, 16384)),
     (12, 12, 64, (1, 63, 64, 97, 129, 300, 2051)),
     (16, 1, 64, (65, 700)),
@@ -89,6 +89,20 @@ def check_batch(gpu, q, kc, vc, n_head, n_head_kv, hd, lengths):
     got = out.download(np.empty_like(q))
     for s, n in enumerate(lengths):
         assert bits_equal(got[s], O.attend(q[s], kc[s, :n], vc[s, :n], n, n_head, n_head_kv, hd)), (s, n)
+
+
+@pytest.mark.parametrize("n_head,n_head_kv,hd,max_kv", [
+    (32, 4, 128, 70), (32, 4, 128, 300), (16, 8, 128, 300), (12, 12, 64, 80), (16, 1, 64, 400)])
+def test_batched_attention_of_few_positions(gpu, n_head, n_head_kv, hd, max_kv):
+    """Sequences of up to 56 positions, which one wave takes with V rows 8 at a
+    time, beside longer ones, whose blocks of logits are shared out over (kv
+    head, sequence) pairs."""
+    lengths = (1, 2, 7, 8, 9, 31, 32, 33, 40, 48, 55, 56, 57, 64, 65, max_kv)
+    kv_dim = n_head_kv * hd
+    q = (H.sample(len(lengths) * n_head * hd, 103) * 3).astype(np.float32).reshape(len(lengths), -1)
+    kc = H.sample(len(lengths) * max_kv * kv_dim, 104).reshape(len(lengths), max_kv, kv_dim)
+    vc = H.sample(len(lengths) * max_kv * kv_dim, 105).reshape(len(lengths), max_kv, kv_dim)
+    check_batch(gpu, q, kc, vc, n_head, n_head_kv, hd, lengths)
 
 
 def test_batched_attention_more_sequences_than_a_grid_dimension(gpu):
