@@ -17,7 +17,7 @@ def bits_equal(a, b):
 
 
 HP_MHA = dict(MF.HP, n_head=4, n_head_kv=4)             # kv groups of one query head
-HP_MHA64 = dict(MF.HP, n_head=8, n_head_kv=8, hd=64)   # hd 64: the three-launch path either way
+HP_MHA64 = dict(MF.HP, n_head=8, n_head_kv=8, hd=64)   # hd 64: never attend_fused
 
 
 @pytest.mark.parametrize("hp,fused,fnorm,nqkv,n_tok", [
@@ -63,14 +63,15 @@ def test_decode_loop_is_bit_identical_to_the_cpu_forward(gpu, tmp_path, hp, fuse
     (MF.HP, 160, -1, 140), (HP_MHA, 160, -1, 140),   # attend_fused throughout
     (MF.HP, 160, 70, 140), (HP_MHA, 160, 70, 140),   # attend_fused, then the split attention
     (MF.HP, 16384, 0, 140), (HP_MHA, 16384, 0, 140),  # split attention throughout
-    (MF.HP, 16384, 300, 400)])   # past the split attention's 320-position V chunks
+    (MF.HP, 16384, 300, 400),
+    (HP_MHA64, 160, 70, 140), (HP_MHA64, 700, 40, 140)])  # heads of 64: attend_decode, then the split attention
 def test_decode_loop_long_context(gpu, tmp_path, hp, max_kv, long_from, n_tok):
     """attend_fused stages cached K and V in LDS 64 positions at a time
-    (chunk boundaries at 64 and 128), and the split attention of long
-    contexts (logits over the whole GPU, then the softmax and the weighted V
-    sum from V chunks in LDS, 320 positions each at max_kv 16384) takes over
-    at long_from, with one and two query heads per kv head. Every token's logits bits and
-    argmax against the CPU forward, across the switch."""
+    (chunk boundaries at 64 and 128), and the split attention (one launch where
+    max_kv is up to 256; else the logits over the whole GPU, then the softmax
+    and the weighted V sum, with the exact sum past 320 positions) takes over at
+    long_from, with one and two query heads per kv head. Every token's logits
+    bits and argmax against the CPU forward, across the switch."""
     from llamd_rs_amd._lib import lib
     from llamd_rs_amd.gguf import Gguf
     p = tmp_path / "tiny.gguf"
