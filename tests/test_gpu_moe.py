@@ -193,8 +193,8 @@ def test_prefill_grouped_equals_token_major(gpu, twin):
 
 def test_prefill_grouping_past_one_id_batch(gpu):
     """The grouping kernel takes the expert ids in batches of 8 per thread of
-    its 1024 (8192 pairs); the last batch stays in registers for the scatter
-    and the others are loaded again. 1040 tokens x top-8 = 8320 pairs cross
+    its 1024; up to 8192 pairs they stay in registers for the scatter, more are
+    loaded again and sorted through LDS. 1040 tokens x top-8 = 8320 pairs cross
     that line: every token is checked bit for bit against the CPU."""
     from llamd_rs_amd import synth
     n_embd, n_ff, n_expert, n_used, n_tok = 512, 256, 16, 8, 1040
